@@ -45,8 +45,8 @@ __device__ __forceinline__ uint32_t calib_word(uint32_t qi, uint32_t ref, uint32
 
 // blockIdx.y: the cycle slice [16 y, 16 y + 16); lane 16 r + j of a step
 // takes cycle 16 y + j of read r, and kCalibUnroll steps load together.  The
-// read store holds (q - q_min) << 2 | base per base, 0 where the base was
-// not observed.
+// read store holds base << 6 | (64 - (q - q_min)) per base, 0 where the base
+// was not observed.
 __global__ __launch_bounds__(kCalibThreads) void k_calib_count(ReadView r, uint64_t n_reads, const uint8_t* ref,
                                                                unsigned long long* hist)
 {

@@ -32,6 +32,10 @@ int guarded(F body)
     }
 }
 struct Ctx;
+// bytes around the read store, so that a wave may load the bytes of a read's
+// row for 64 consecutive sites whether the read covers them or not: at most
+// 63 before the row and 63 + 255 after its start
+constexpr size_t kSeqFront = 64, kSeqBack = 512;
 // calibration bins: (q - q_min) << 12 | cycle << 4 | ref << 2 | obs
 constexpr uint32_t kCalibBins = 64u << 12;
 int dict_encode_device(Ctx& c, const int32_t* d_in, uint64_t n, uint64_t* n_words, uint64_t* n_dict);
@@ -209,7 +213,8 @@ struct ChromState {
     uint32_t pitch = 0;
     DevBuf<int32_t> rpos;
     DevBuf<uint32_t> rmeta;
-    DevBuf<uint8_t> rseq;
+    DevBuf<uint64_t> rfirst;  // first read at or after each kReadBlock sites
+    DevBuf<uint8_t> rseq;  // kSeqFront bytes, the packed reads, kSeqBack bytes
     std::vector<int32_t> h_rpos;
     std::vector<gsnp_snp> h_snps;
     std::vector<uint8_t> h_snp_ref;
@@ -253,11 +258,20 @@ struct Ctx {
     int device = 0;  // HIP device current when the context was created
     hipStream_t stream = nullptr;      // where the context's work is queued
     hipStream_t own_stream = nullptr;  // the stream the context created (stream unless a caller's is set)
+    // a span's deepest tiles run beside its others
+    hipStream_t side = nullptr;
+    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     StageTimer timer;
     // tables
     DevBuf<double> score, lprior, prank;
     DevBuf<uint8_t> qadj;
     int td = 1, gd = 1;
+    // the tile form of both (call.hip): qadj by 64 - q, the score rows of
+    // adjusted qualities below 64 by base; tile_ok when they hold every value
+    DevBuf<uint8_t> qtab;
+    DevBuf<double> tscore;
+    uint32_t qtab_bytes = 0;
+    bool tile_ok = false;
     std::vector<double> h_prank, h_pprior;
     // chromosome (the fields of ChromState; chrom_id names the uploaded
     // inputs in the keys of captured graphs)
@@ -274,6 +288,7 @@ struct Ctx {
     uint32_t pitch = 0;
     DevBuf<int32_t> rpos;
     DevBuf<uint32_t> rmeta;
+    DevBuf<uint64_t> rfirst;
     DevBuf<uint8_t> rseq;
     std::vector<int32_t> h_rpos;
     // sites of the current window (or batched span)
@@ -364,6 +379,7 @@ struct Ctx {
     int span_build(uint32_t start, uint32_t n);
     int span_prepare(uint32_t n);
     void span_enqueue(uint32_t start, uint32_t n);
+    void span_enqueue_tiles(uint32_t start, uint32_t n);
     template <class F>
     int launch_captured(GraphSlot& slot, const std::vector<uint64_t>& key, F enqueue);
     FusedArgs fused_args(uint32_t start);

@@ -190,7 +190,8 @@ ReadView Ctx::read_view() const
     ReadView v;
     v.pos = rpos.p;
     v.meta = rmeta.p;
-    v.seq = rseq.p;
+    v.first = rfirst.p;
+    v.seq = rseq.p ? rseq.p + kSeqFront : nullptr;
     v.pitch = pitch ? pitch : 1u;
     return v;
 }
@@ -300,6 +301,7 @@ void Ctx::swap_chrom(ChromState& s)
     std::swap(pitch, s.pitch);
     rpos.swap(s.rpos);
     rmeta.swap(s.rmeta);
+    rfirst.swap(s.rfirst);
     rseq.swap(s.rseq);
     h_rpos.swap(s.h_rpos);
     h_snps.swap(s.h_snps);
@@ -322,6 +324,11 @@ int Ctx::set_matrix(const double* p_matrix)
     HIPCHK(hipStreamSynchronize(stream));
     if (score.n != sc.size()) HIPCHK(score.alloc(sc.size()));
     HIPCHK(hipMemcpyAsync(score.p, sc.data(), sc.size() * 8, hipMemcpyHostToDevice, stream));
+    if (tile_ok) {
+        if (!tscore.p) HIPCHK(tscore.alloc((size_t)4 * 64 * p.read_length * kScoreRowStride));
+        launch_tile_scores(stream, score.p, tscore.p, (uint32_t)p.read_length);
+        HIPCHK(hipGetLastError());
+    }
     HIPCHK(hipStreamSynchronize(stream));
     return GSNP_OK;
 }
@@ -339,6 +346,9 @@ int create_ctx(const gsnp_params* p, const double* p_matrix, gsnp_ctx** out)
     HIPCHK(hipGetDevice(&c->device));
     HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     c->own_stream = c->stream;
+    HIPCHK(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
+    HIPCHK(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
+    HIPCHK(hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
     // adjusted qualities, priors, rank table (the score table: set_matrix)
     QadjTable qt = build_qadj_table(p->pcr_dependency, p->global_dependency);
     c->td = qt.td;
@@ -347,11 +357,16 @@ int create_ctx(const gsnp_params* p, const double* p_matrix, gsnp_ctx** out)
     prior_gen(*p, c->h_pprior.data());
     std::vector<double> lp = log_prior_rows(c->h_pprior.data());
     c->h_prank = rank_table();
+    const std::vector<uint8_t> tq = tile_qadj(qt);
+    c->tile_ok = !tq.empty() && tq.size() <= kTileQtabMax;
+    c->qtab_bytes = c->tile_ok ? (uint32_t)tq.size() : 0u;
+    HIPCHK(c->qtab.alloc(tq.size()));
+    if (c->tile_ok) HIPCHK(hipMemcpyAsync(c->qtab.p, tq.data(), tq.size(), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c->qadj.alloc(qt.v.size()));
     HIPCHK(c->lprior.alloc(lp.size()));
     HIPCHK(c->prank.alloc(c->h_prank.size()));
     HIPCHK(c->err.alloc(1));
-    HIPCHK(c->counts.alloc(8));
+    HIPCHK(c->counts.alloc(8 * kCountStride));
     HIPCHK(c->job_count.alloc(1));
     HIPCHK(c->fix_count.alloc(1));
     HIPCHK(c->total.alloc(1));
@@ -417,8 +432,12 @@ void gsnp_destroy(gsnp_ctx* c)
 {
     if (!c) return;
     if (c->stream) hipStreamSynchronize(c->stream);
-    hipStream_t s = c->own_stream;
+    hipStream_t s = c->own_stream, side = c->side;
+    if (side) (void)hipStreamSynchronize(side);
+    for (hipEvent_t e : {c->ev_fork, c->ev_join})
+        if (e) (void)hipEventDestroy(e);
     delete c;
+    if (side) (void)hipStreamDestroy(side);
     if (s) hipStreamDestroy(s);
 }
 
@@ -502,7 +521,7 @@ int gsnp_load_reads(gsnp_ctx* c, const gsnp_read_batch* b)
     const uint32_t L = (uint32_t)c->p.read_length;
     if (b->n && (b->pitch < 1 || !b->pos || !b->len_hit || !b->strand || !b->seq || !b->qual))
         return fail(GSNP_E_ARG, "incomplete read batch");
-    // validate and pack: byte = (q << 2) | base, 0 when the base is not observed;
+    // validate and pack: byte = (base << 6) | (64 - q), 0 when the base is not observed;
     // ranges of reads on threads, the error of the lowest read index reported
     std::vector<uint32_t> meta(b->n);
     std::unique_ptr<uint8_t[]> seq(new uint8_t[(size_t)b->n * L + 1]);
@@ -550,7 +569,7 @@ int gsnp_load_reads(gsnp_ctx* c, const gsnp_read_batch* b)
                 } else {
                     qq = 1;  // repeats only count the base; any non-zero quality marks it observed
                 }
-                o[k] = (uint8_t)((qq << 2) | (((unsigned)sq[k] >> 1) & 3));
+                o[k] = (uint8_t)pb_encode(((unsigned)sq[k] >> 1) & 3, qq);
             }
         }
     };
@@ -582,12 +601,22 @@ int gsnp_load_reads(gsnp_ctx* c, const gsnp_read_batch* b)
     c->h_rpos.assign(b->pos, b->pos + b->n);
     HIPCHK(c->rpos.alloc(b->n + 1));
     HIPCHK(c->rmeta.alloc(b->n + 1));
+    // first read at or after each block of sites (the tiles' range searches)
+    const size_t nfirst = (size_t)(chr_len / kReadBlock) + 3;
+    std::vector<uint64_t> first(nfirst);
+    uint64_t at = 0;
+    for (size_t k = 0; k < nfirst; k++) {
+        while (at < b->n && (uint64_t)b->pos[at] < (uint64_t)k * kReadBlock) at++;
+        first[k] = at;
+    }
+    HIPCHK(c->rfirst.alloc(nfirst));
+    HIPCHK(hipMemcpyAsync(c->rfirst.p, first.data(), 8 * nfirst, hipMemcpyHostToDevice, c->stream));
     const size_t nseq = (size_t)b->n * L;
-    HIPCHK(c->rseq.alloc(nseq + 64));
+    HIPCHK(c->rseq.alloc(kSeqFront + nseq + kSeqBack));
     if (b->n) {
         HIPCHK(hipMemcpyAsync(c->rpos.p, b->pos, 4 * b->n, hipMemcpyHostToDevice, c->stream));
         HIPCHK(hipMemcpyAsync(c->rmeta.p, meta.data(), 4 * b->n, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(hipMemcpyAsync(c->rseq.p, seq.get(), nseq, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(hipMemcpyAsync(c->rseq.p + kSeqFront, seq.get(), nseq, hipMemcpyHostToDevice, c->stream));
     }
     HIPCHK(hipStreamSynchronize(c->stream));
     c->n_reads = b->n;
@@ -931,6 +960,10 @@ int Ctx::span_prepare(uint32_t n)
 // only (no copies, no memsets, no host waits), so it can be captured.
 void Ctx::span_enqueue(uint32_t start, uint32_t n)
 {
+    if (tile_ok) {
+        span_enqueue_tiles(start, n);
+        return;
+    }
     launch_fill_u32(stream, head_qs.p, (uint32_t)(4 * (n / GSNP_WIN + 2)), 0u);
     timer.begin(kStSiteBuild, stream);
     launch_site_build(stream, read_view(), 0, n_reads, start, n + 1, INT64_MIN, (int64_t)start + n, 0, site_view(0),
@@ -949,6 +982,62 @@ void Ctx::span_enqueue(uint32_t start, uint32_t n)
         Results res = result_view(0);
         timer.begin(kStRank, stream);
         launch_rank(stream, tables(), a, jobs.p, job_count.p, n, res, fixes.p, fix_count.p, stat.p + 1);
+        timer.end(kStRank, stream);
+    }
+}
+
+// The same through the tile kernels (call.hip): classes of the span's tiles,
+// reads to calls per class, then the few tiles deeper than those classes.
+void Ctx::span_enqueue_tiles(uint32_t start, uint32_t n)
+{
+    const uint32_t n_tiles = (n + 1 + 63) / 64;  // one more site is built: the last one's next
+    SpanClear clr;
+    clr.head_qs = head_qs.p;
+    clr.n_heads = n / GSNP_WIN + 2;
+    clr.counts = counts.p;
+    clr.job_count = job_count.p;
+    clr.fix_count = fix_count.p;
+    timer.begin(kStBucket, stream);
+    launch_tile_classes(stream, read_view(), start, n_tiles, ranges.p, lists.p, n_tiles, clr);
+    timer.end(kStBucket, stream);
+    TileArgs f;
+    f.t = tables();
+    f.ref = ref_view();
+    f.reads = read_view();
+    f.range = ranges.p;
+    f.qtab = qtab.p;
+    f.qtab_bytes = qtab_bytes;
+    f.score = tscore.p;
+    f.ws = start;
+    f.n_sites = n;
+    f.n_built = n + 1;
+    f.a = site_view(0);
+    f.head_qs = head_qs.p;
+    f.out = result_view(0);
+    f.jobs = jobs.p;
+    f.job_count = job_count.p;
+    f.n_records = stat.p;
+    f.write_lk = keep_lk ? 1 : 0;
+    timer.begin(kStFused, stream);
+    // the deepest tiles are few and long: beside the others, unless those are
+    // few as well (a fork and join costs about as much as their launch)
+    const bool fork = n_tiles > 2048;
+    if (fork) {
+        (void)hipEventRecord(ev_fork, stream);
+        (void)hipStreamWaitEvent(side, ev_fork, 0);
+    }
+    launch_call_deepest(fork ? side : stream, f, lists.p, n_tiles, counts.p, n_tiles);
+    if (fork) (void)hipEventRecord(ev_join, side);
+    launch_call_tiles(stream, f, lists.p, n_tiles, counts.p, n_tiles);
+    if (fork) (void)hipStreamWaitEvent(stream, ev_join, 0);
+    launch_deep_tiles(stream, fused_args(start), read_view(), ranges.p, n + 1, n, head_qs.p,
+                      lists.p + (size_t)kTileClasses * n_tiles, counts.p + kTileClasses * kCountStride, lists.p + 5 * (size_t)win_cap,
+                      counts.p + (kTileClasses + 1) * kCountStride, n_tiles, stat.p);
+    timer.end(kStFused, stream);
+    if (p.rank_sum_mode) {
+        Results res = result_view(0);
+        timer.begin(kStRank, stream);
+        launch_rank(stream, tables(), site_view(0), jobs.p, job_count.p, n, res, fixes.p, fix_count.p, stat.p + 1);
         timer.end(kStRank, stream);
     }
 }

@@ -32,10 +32,12 @@ GSNP_HD uint32_t rec_strand(uint32_t w) { return (w & 0x00000100u) >> 8; }
 GSNP_HD uint32_t rec_occ(uint32_t w) { return w & 0xffu; }
 GSNP_HD uint32_t rec_key(uint32_t w) { return (w >> 8) & 0x1ffu; }  // (cycle, strand)
 
-// Packed read base byte: (q << 2) | base, with 0 meaning "not observed"
-// (N, non-ACGT, or quality below q_min).  q is in [1, 63].
-GSNP_HD uint32_t pb_base(uint32_t b) { return b & 3u; }
-GSNP_HD uint32_t pb_q(uint32_t b) { return b >> 2; }
+// Packed read base byte: (base << 6) | (64 - q), the record's base and quality
+// fields as they stand in bits 24:17, with 0 meaning "not observed" (N,
+// non-ACGT, or quality below q_min).  q is in [1, 63].
+GSNP_HD uint32_t pb_encode(uint32_t base, uint32_t q) { return (base << 6) | (64u - q); }
+GSNP_HD uint32_t pb_base(uint32_t b) { return b >> 6; }
+GSNP_HD uint32_t pb_q(uint32_t b) { return 64u - (b & 63u); }
 
 // Read metadata word: bits 15:0 hit, 24:16 length (1..256), 31 strand ('-').
 GSNP_HD uint32_t rm_hit(uint32_t m) { return m & 0xffffu; }

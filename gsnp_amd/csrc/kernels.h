@@ -40,7 +40,9 @@ struct RefView {
     const uint32_t* snp_first = nullptr;  // [len/256 + 2]: first known SNP at or after each 256-site block
 };
 
+constexpr uint32_t kReadBlock = 1024;  // sites per entry of ReadView::first
 struct ReadView {
+    const uint64_t* first = nullptr;  // [len / kReadBlock + 3]: first read at or after each block of sites
     const int32_t* pos = nullptr;
     const uint32_t* meta = nullptr;
     const uint8_t* seq = nullptr;
@@ -113,6 +115,55 @@ struct FusedTune {
     uint32_t wpb[6] = {0, 4, 8, 8, 4, 4};
     uint32_t max_blocks[6] = {8192, 8192, 8192, 8192, 8192, 8192};
 };
+
+// Counters that many blocks add to lie this many words apart.
+constexpr uint32_t kCountStride = 64;
+
+// Arguments of the reads-to-calls launch over tiles of 64 sites (call.hip).
+constexpr uint32_t kTileClasses = 5;         // at most 16, 32, 40, 64, 128 records a site; then the deep tiles
+constexpr uint32_t kTileQtabMax = 17408;     // bytes of the adjusted-quality table that fit beside the waves' LDS
+struct TileArgs {
+    Tables t;
+    RefView ref;
+    ReadView reads;
+    const uint64_t* range = nullptr;  // reads of each tile
+    const uint8_t* qtab = nullptr;    // [64 - q][td][gd], 16-byte aligned; row 0 (empty slots) all 0
+    uint32_t qtab_bytes = 0;          // a multiple of 16, at most kTileQtabMax
+    const double* score = nullptr;    // [base][adjusted quality < 64][cycle < read length][16]
+    uint32_t ws = 0;
+    uint32_t n_sites = 0;   // sites called
+    uint32_t n_built = 0;   // sites whose counters are stored (one more)
+    SiteArrays a;
+    int4* head_qs = nullptr;
+    Results out;
+    RankJob* jobs = nullptr;
+    uint32_t* job_count = nullptr;
+    unsigned long long* n_records = nullptr;
+    int write_lk = 0;
+};
+// what the first launch of a span clears: window heads, class counters (8, kCountStride words apart), job counters
+struct SpanClear {
+    int4* head_qs = nullptr;
+    uint32_t n_heads = 0;
+    uint32_t* counts = nullptr;
+    uint32_t *job_count = nullptr, *fix_count = nullptr;
+};
+// reads, class and class list (lists[class * pitch]) of each tile of 64 sites
+void launch_tile_classes(hipStream_t s, const ReadView& r, uint32_t ws, uint32_t n_tiles, uint64_t* range,
+                         uint32_t* lists, uint32_t pitch, const SpanClear& clr);
+// the deepest class, a few long tiles, and the others
+void launch_call_deepest(hipStream_t s, const TileArgs& f, const uint32_t* lists, uint32_t pitch,
+                         const uint32_t* counts, uint32_t n_tiles);
+void launch_call_tiles(hipStream_t s, const TileArgs& f, const uint32_t* lists, uint32_t pitch, const uint32_t* counts,
+                       uint32_t n_tiles);
+// the tiles beyond those classes: site matrix, then every called site of them
+// sorted and called by the 256-record network
+void launch_deep_tiles(hipStream_t s, const FusedArgs& f, const ReadView& r, const uint64_t* range, uint32_t n_built,
+                       uint32_t n_sites, int4* head_qs, const uint32_t* tiles, const uint32_t* n_deep, uint32_t* sites,
+                       uint32_t* site_count, uint32_t n_tiles, unsigned long long* n_records);
+
+// score rows [base][adjusted quality < 64][cycle] from the table by quality, cycle, base
+void launch_tile_scores(hipStream_t s, const double* score, double* tscore, uint32_t cycles);
 
 void launch_fill_u32(hipStream_t s, void* p, uint32_t n_words, uint32_t v);
 

@@ -8,6 +8,7 @@
 #include "gsnp_common.h"
 #include "kernels.h"
 #include "nearest.h"
+#include "posterior.h"
 #include "walk.h"
 
 namespace gsnp {
@@ -78,18 +79,27 @@ __global__ __launch_bounds__(256) void k_read_ranges(const int32_t* pos, uint64_
     range[2 * blk + 1] = e;
 }
 
-__global__ __launch_bounds__(kBuildSites) void k_site_build(ReadView r, const uint64_t* range, uint32_t ws, uint32_t n_sites,
-                                                    uint32_t carry, SiteArrays a, int4* head_qs)
+struct BuildLds {
+    __align__(16) uint8_t seq[kStageBytes + 32];
+    int32_t pos[kStageReads];
+    uint32_t meta[kStageReads];
+    int ca[4 * kBuildSites];  // count_all, one LDS add per observed base
+};
+
+// Sites [64 * tile, 64 * tile + 64); returns the records of the thread's site (0 beyond the span).
+__device__ __forceinline__ int build_tile(const ReadView& r, const uint64_t* range, uint32_t ws, uint32_t n_sites,
+                                          uint32_t carry, const SiteArrays& a, int4* head_qs, uint32_t tile,
+                                          BuildLds& sh)
 {
-    __shared__ __align__(16) uint8_t sseq[kStageBytes + 32];
-    __shared__ int32_t spos[kStageReads];
-    __shared__ uint32_t smeta[kStageReads];
-    __shared__ int sca[4 * kBuildSites];  // count_all, one LDS add per observed base
-    const uint32_t s = blockIdx.x * kBuildSites + threadIdx.x;
+    uint8_t* sseq = sh.seq;
+    int32_t* spos = sh.pos;
+    uint32_t* smeta = sh.meta;
+    int* sca = sh.ca;
+    const uint32_t s = tile * kBuildSites + threadIdx.x;
     const uint32_t pitch = r.pitch;
     const uint32_t kr = kStageBytes / pitch < kStageReads ? kStageBytes / pitch : kStageReads;
     // block-uniform bounds: keep the read loop on scalar registers
-    const uint64_t rb = range[2 * blockIdx.x], re = range[2 * blockIdx.x + 1];
+    const uint64_t rb = range[2 * tile], re = range[2 * tile + 1];
     const uint64_t b = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(rb >> 32)) << 32) |
                        (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)rb);
     const uint64_t e = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(re >> 32)) << 32) |
@@ -126,7 +136,7 @@ __global__ __launch_bounds__(kBuildSites) void k_site_build(ReadView r, const ui
     sca[2 * kBuildSites + threadIdx.x] = ca2;
     sca[3 * kBuildSites + threadIdx.x] = ca3;
     const int64_t p = (int64_t)ws + s;
-    const int64_t p0 = (int64_t)ws + (int64_t)blockIdx.x * kBuildSites;  // the block's first site
+    const int64_t p0 = (int64_t)ws + (int64_t)tile * kBuildSites;  // the block's first site
     const int32_t lane = (int32_t)threadIdx.x;
     const bool head = head_qs && live && (p % kWin) == 0;
     const bool any_head = __ballot(head) != 0;  // block-uniform: the snapshot test leaves the read loop of other blocks
@@ -184,7 +194,7 @@ __global__ __launch_bounds__(kBuildSites) void k_site_build(ReadView r, const ui
             atomicAdd(&sca[o * kBuildSites + threadIdx.x], 1);
         }
     }
-    if (!live) return;
+    if (!live) return 0;
     if (const int k = nrec & 3) {  // the last k records, left-aligned
         const uint32_t x = k == 1 ? pb3 : k == 2 ? pb2 : pb1;
         *reinterpret_cast<uint4*>(row + (nrec & ~3)) = make_uint4(x, k == 2 ? pb3 : pb2, pb3, 0u);
@@ -199,6 +209,41 @@ __global__ __launch_bounds__(kBuildSites) void k_site_build(ReadView r, const ui
     a.qs[s] = make_int4((int)(qs & 0xffff), (int)((qs >> 16) & 0xffff), (int)((qs >> 32) & 0xffff), (int)(qs >> 48));
     a.ca[s] = make_int4(sca[0 * kBuildSites + threadIdx.x], sca[1 * kBuildSites + threadIdx.x],
                         sca[2 * kBuildSites + threadIdx.x], sca[3 * kBuildSites + threadIdx.x]);
+    return nrec;
+}
+
+__global__ __launch_bounds__(kBuildSites) void k_site_build(ReadView r, const uint64_t* range, uint32_t ws, uint32_t n_sites,
+                                                    uint32_t carry, SiteArrays a, int4* head_qs)
+{
+    __shared__ BuildLds sh;
+    build_tile(r, range, ws, n_sites, carry, a, head_qs, blockIdx.x, sh);
+}
+
+// The same for the listed tiles of a span, whose called sites go to the site list of k_fused.
+__global__ __launch_bounds__(kBuildSites) void k_site_build_list(ReadView r, const uint64_t* range, uint32_t ws,
+                                                                 uint32_t n_built, uint32_t n_sites, SiteArrays a,
+                                                                 int4* head_qs, const uint32_t* tiles,
+                                                                 const uint32_t* n_tiles, uint32_t* sites,
+                                                                 uint32_t* site_count, unsigned long long* n_records)
+{
+    __shared__ BuildLds sh;
+    const uint32_t count = *n_tiles;
+    for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {
+        const uint32_t tile = tiles[i];
+        const int n = build_tile(r, range, ws, n_built, 0, a, head_qs, tile, sh);
+        const uint32_t s = tile * kBuildSites + threadIdx.x;
+        const uint64_t called = __ballot(s < n_sites);  // the tile's first lanes
+        unsigned long long recs = s < n_sites ? (unsigned long long)n : 0ull;
+        for (int off = 32; off > 0; off >>= 1) recs += __shfl_xor(recs, off);
+        uint32_t base = 0;
+        if (threadIdx.x == 0) {
+            base = atomicAdd(site_count, (uint32_t)__popcll(called));
+            if (recs) atomicAdd(n_records, recs);
+        }
+        base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+        if (s < n_sites) sites[base + threadIdx.x] = s;
+        __syncthreads();
+    }
 }
 
 void launch_site_build(hipStream_t st, const ReadView& r, uint64_t r0, uint64_t r1, uint32_t ws, uint32_t n_sites,
@@ -563,146 +608,28 @@ void launch_likelihood(hipStream_t st, const Tables& t, const SiteArrays& a, uin
 // (reference code rows, or a known-SNP row found by binary search).  A het
 // call under the rank-sum mode is handed to k_rank through a job list.
 
-__device__ __forceinline__ int get4(const int4& v, uint32_t i)
-{
-    return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
-}
-
-// Calls site s from its ten log-likelihoods lkv(0..9).
+// Calls site s from its ten log-likelihoods lkv(0..9) and its counters in memory.
 template <class LK>
 __device__ __forceinline__ void posterior_site(const Tables& t, const RefView& ref, uint32_t ws, const SiteArrays& a,
                                                uint32_t s, LK lkv, const int4* head_qs, const Results& out,
                                                RankJob* jobs, uint32_t* job_count)
 {
-    const uint32_t ori = ref.code[ws + s] & 0xF;
-    const int depth = a.depth[s];
-    if ((ori & 4) && depth == 0) return;  // N row, not called (nflag)
-    const int dep_uni = a.nrec[s];
-    const int4 qs = a.qs[s];
-    const int4 ca = a.ca[s];
-    // base1/base2 and qual1..3 (>= keeps the later base on ties)
-    uint32_t base1 = 0, base2 = 0;
-    int qual1 = -1, qual2 = -2, qual3 = -3;
-    const int4 key = dep_uni ? qs : ca;
-    int k1 = dep_uni ? -1 : 0, k2 = dep_uni ? -2 : 0, k3 = dep_uni ? -3 : 0;
-#pragma unroll
-    for (uint32_t i = 0; i < 4; i++) {
-        const int v = get4(key, i);
-        if (v >= k1) {
-            k3 = k2;
-            base2 = base1;
-            k2 = k1;
-            base1 = i;
-            k1 = v;
-        } else if (v >= k2) {
-            k3 = k2;
-            base2 = i;
-            k2 = v;
-        } else if (v >= k3) {
-            k3 = v;
-        }
+    SiteVals v;
+    v.ori = ref.code[ws + s] & 0xF;
+    v.depth = a.depth[s];
+    if ((v.ori & 4) && v.depth == 0) return;  // N row, not called (nflag)
+    v.dep_uni = a.nrec[s];
+    v.qs = a.qs[s];
+    v.ca = a.ca[s];
+    v.cu = t.rank_mode ? a.cu[s] : make_int4(0, 0, 0, 0);  // read by the rank-sum mode only
+    const double* lp = t.lprior + (v.ori & 7) * 10;
+    const SiteCall c = call_site(t, ref, ws + s, v, lkv, [&](int g) { return lp[g]; });
+    int4 nq = v.qs;
+    if (c.next) {  // head_qs: the batched span's window heads before their own reads
+        const uint32_t nx = ws + s + 1;
+        nq = (head_qs && nx % kWin == 0) ? head_qs[nx / kWin - ws / kWin] : a.qs[s + 1];
     }
-    if (k1 == 0)
-        base1 = ori & 7;
-    else if (k2 == 0 && base1 != (ori & 7))
-        base2 = ori & 7;
-    if (dep_uni) {
-        qual1 = k1;
-        qual2 = k2;
-        qual3 = k3;
-    }
-    // log10 priors
-    const double* lp = t.lprior + (ori & 7) * 10;
-    if ((ori & 8) && t.refine && ref.n_snp) {
-        // the known SNPs of the site's 256-site block, then a search among them
-        const uint32_t p = ws + s;
-        uint32_t lo = ref.snp_first[p >> 8], hi = ref.snp_first[(p >> 8) + 1];
-        while (lo < hi) {
-            uint32_t m = (lo + hi) >> 1;
-            if (ref.snp_pos[m] < p)
-                lo = m + 1;
-            else
-                hi = m;
-        }
-        if (lo < ref.n_snp && ref.snp_pos[lo] == p) lp = ref.snp_lp + (size_t)lo * 10;
-    }
-    uint32_t type1 = 16, type2 = 16;
-    double tp1 = 0.0, tp2 = 0.0;
-#pragma unroll
-    for (int g = 0; g < 10; g++) {
-        const uint32_t gt = geno_code(g);
-        if (t.monoploid && (gt >> 2) != (gt & 3)) continue;
-        const double v = lkv(g) + lp[g];
-        if (v >= tp1 || type1 == 16) {
-            type2 = type1;
-            tp2 = tp1;
-            type1 = gt;
-            tp1 = v;
-        } else if (v >= tp2 || type2 == 16) {
-            type2 = gt;
-            tp2 = v;
-        }
-    }
-    const double dtp = tp1 - tp2;
-    const bool hom = (type1 & 3) == ((type1 >> 2) & 3);
-    // HET cap inputs; q_sum is flat over sites, so base codes 4..7 read the next
-    // site -- for the last site of a window, as it stands before the reads
-    // that start on the window boundary (head_qs in the batched span)
-    bool het_ok = false;
-    if (!hom) {
-        const uint32_t het = base1 < base2 ? (base1 << 2 | base2) : (base2 << 2 | base1);
-        int4 nq = qs;
-        if (base1 >= 4 || base2 >= 4) {
-            const uint32_t nx = ws + s + 1;
-            nq = (head_qs && nx % kWin == 0) ? head_qs[nx / kWin - ws / kWin] : a.qs[s + 1];
-        }
-        const int q_b1 = base1 < 4 ? get4(qs, base1) : get4(nq, base1 & 3);
-        const int q_b2 = base2 < 4 ? get4(qs, base2) : get4(nq, base2 & 3);
-        het_ok = q_b1 > 0 && q_b2 > 0 && type1 == het;
-    }
-    double rank = 1.0;
-    int q_cns;
-    if (t.rank_mode && !hom) {
-        const int4 cu = a.cu[s];
-        if (get4(cu, type1 & 3) == 0 || get4(cu, (type1 >> 2) & 3) == 0) {
-            rank = 0.0;
-        } else {
-            const uint32_t j = atomicAdd(job_count, 1u);
-            // written as three words (a struct copy with byte fields would go through scratch)
-            uint32_t* jw = reinterpret_cast<uint32_t*>(jobs + j);
-            jw[0] = s;
-            jw[1] = (type1 & 0xffu) | ((het_ok ? 1u : 0u) << 8);
-            jw[2] = (uint32_t)(qual2 - qual3);
-            jobs[j].dtp = dtp;
-            out.base1[s] = (uint8_t)base1;
-            out.base2[s] = (uint8_t)base2;
-            out.type1[s] = (uint8_t)type1;
-            return;  // rank and q_cns come from k_rank
-        }
-    }
-    if (rank == 0.0)
-        q_cns = 0;
-    else
-        q_cns = trunc_int_x86(10 * dtp + 0.0);  // 10*log10(1) == 0
-    if (hom) {
-        if (qual1 > 0 && base1 != (type1 & 3))
-            q_cns = 0;
-        else if (q_cns > qual1 - qual2)
-            q_cns = qual1 - qual2;
-    } else {
-        if (het_ok) {
-            if (q_cns > qual2 - qual3) q_cns = qual2 - qual3;
-        } else {
-            q_cns = 0;
-        }
-    }
-    if (q_cns > 99) q_cns = 99;
-    if (q_cns < 0) q_cns = 0;
-    out.base1[s] = (uint8_t)base1;
-    out.base2[s] = (uint8_t)base2;
-    out.type1[s] = (uint8_t)type1;
-    out.q_cns[s] = q_cns;
-    out.rank[s] = rank;
+    finish_site(t, v, c, nq, s, out, jobs, job_count);
 }
 
 __global__ __launch_bounds__(256) void k_posterior(Tables t, RefView ref, uint32_t ws, SiteArrays a, uint32_t n_sites,
@@ -1174,6 +1101,18 @@ void launch_fused(hipStream_t st, const FusedArgs& f, const uint32_t* lists, uin
     // deepest classes first: their groups are the longest
     for (int cls = 5; cls >= (int)tune.min_class; cls--)
         launch_fused_one(st, f, lists, pitch, counts, max_sites, (uint32_t)cls, tune.wpb[cls], tune.max_blocks[cls]);
+}
+
+void launch_deep_tiles(hipStream_t st, const FusedArgs& f, const ReadView& r, const uint64_t* range, uint32_t n_built,
+                       uint32_t n_sites, int4* head_qs, const uint32_t* tiles, const uint32_t* n_deep, uint32_t* sites,
+                       uint32_t* site_count, uint32_t n_tiles, unsigned long long* n_records)
+{
+    if (!n_tiles) return;
+    // few tiles are this deep, so the grids stay small and loop
+    const uint32_t blocks = n_tiles < 2048u ? n_tiles : 2048u;
+    hipLaunchKernelGGL(k_site_build_list, dim3(blocks), dim3(kBuildSites), 0, st, r, range, f.ws, n_built, n_sites, f.a,
+                       head_qs, tiles, n_deep, sites, site_count, n_records);
+    launch_fused_class<256>(st, f, sites, site_count, n_sites, 0, 1024u);
 }
 
 // ---------------------------------------------------------------------------

@@ -74,6 +74,19 @@ QadjTable build_qadj_table(double pcr, double glob)
     return t;
 }
 
+std::vector<uint8_t> tile_qadj(const QadjTable& t)
+{
+    const size_t row = (size_t)t.td * t.gd;
+    std::vector<uint8_t> v((64 * row + 15) / 16 * 16, 0);
+    for (int q = 1; q < 64; q++)
+        for (size_t i = 0; i < row; i++) {
+            const uint8_t qa = t.v[q * row + i];
+            if (qa < 1 || qa > 63) return {};
+            v[(64 - q) * row + i] = qa;
+        }
+    return v;
+}
+
 void prior_gen(const gsnp_params& p, double* pp)
 {
     for (int i = 0; i < 128; i++) pp[i] = 1.0;

@@ -26,6 +26,10 @@ struct QadjTable {
 };
 QadjTable build_qadj_table(double pcr, double glob);
 
+// The table by 64 - q (row 0 all 0), padded to 16 bytes; empty when a value
+// of q in [1,64) is above 63.
+std::vector<uint8_t> tile_qadj(const QadjTable& t);
+
 // Genotype priors p_prior[ref(8)][a1<<2|a2] (cpp/prior.cc:3-43).
 void prior_gen(const gsnp_params& p, double* p_prior /*128*/);
 
