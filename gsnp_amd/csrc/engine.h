@@ -131,23 +131,6 @@ struct StageTimer {
     ~StageTimer();
 };
 
-// An instantiated graph of a captured launch sequence and the key (shape and
-// buffer generation) it was captured for.
-struct GraphSlot {
-    hipGraphExec_t exec = nullptr;
-    std::vector<uint64_t> key;
-    GraphSlot() = default;
-    GraphSlot(const GraphSlot&) = delete;
-    GraphSlot& operator=(const GraphSlot&) = delete;
-    void reset()
-    {
-        if (exec) (void)hipGraphExecDestroy(exec);
-        exec = nullptr;
-        key.clear();
-    }
-    ~GraphSlot() { reset(); }
-};
-
 // Device buffers of the -C column encoder, sized for `win` windows of
 // GSNP_WIN sites (segment w of each per-window array starts at w*GSNP_WIN).
 struct ColBufs {
@@ -274,7 +257,7 @@ struct Ctx {
     bool tile_ok = false;
     std::vector<double> h_prank, h_pprior;
     // chromosome (the fields of ChromState; chrom_id names the uploaded
-    // inputs in the keys of captured graphs)
+    // inputs, 0: none)
     uint64_t chrom_id = 0;
     std::string chr_name;
     uint32_t chr_len = 0;
@@ -318,13 +301,6 @@ struct Ctx {
     DevBuf<GText> gtext;
     bool keep_lk = false;     // batched form: also store the per-site log-likelihoods
     FusedTune tune;           // launch shape of the fused stage (gsnp_autotune)
-    // batched span and its formatting replay as graphs while shape and buffers
-    // stay the same; buf_gen counts buffer (re)allocations and chromosome or
-    // read changes, each made after a stream sync, and drops the cached graphs
-    bool use_graphs = true;
-    uint64_t buf_gen = 0, graphs_gen = 0;
-    std::vector<std::unique_ptr<GraphSlot>> graphs;  // captured spans, at most kMaxGraphs
-    GraphSlot& graph_slot(const std::vector<uint64_t>& key);
     DevBuf<char> text;  // rows of the per-window path and of spans formatted for gsnp_fetch_text
     uint64_t text_cap = 0, text_len = 0;
     TextPipe pipe;      // rows of batched spans copied to host memory (gsnp_job_call, gsnp_run)
@@ -375,13 +351,11 @@ struct Ctx {
     int host_fixups();
     int check_err();
     int format_text(uint32_t offset, uint32_t ws_abs, uint32_t n_sites, uint32_t pos_base, uint64_t* nbytes,
-                    bool graph = false, char* out = nullptr);
+                    char* out = nullptr);
     int span_build(uint32_t start, uint32_t n);
     int span_prepare(uint32_t n);
     void span_enqueue(uint32_t start, uint32_t n);
     void span_enqueue_tiles(uint32_t start, uint32_t n);
-    template <class F>
-    int launch_captured(GraphSlot& slot, const std::vector<uint64_t>& key, F enqueue);
     FusedArgs fused_args(uint32_t start);
 };
 

@@ -95,7 +95,6 @@ int Ctx::alloc_window(uint32_t n_sites)
 {
     if (n_sites <= win_cap) return GSNP_OK;
     HIPCHK(hipStreamSynchronize(stream));  // nothing queued may still use the old buffers
-    buf_gen++;
     sites.reset();
     win_cap = 0;
     const size_t n = n_sites;
@@ -468,7 +467,6 @@ int gsnp_set_chromosome(gsnp_ctx* c, const char* name, const uint8_t* codes, uin
     c->chr_len = 0;
     c->n_snp = 0;
     c->n_reads = 0;
-    c->buf_gen++;
     c->chrom_id = next_chrom_id();
     c->chr_name = name;
     HIPCHK(c->ref.alloc((size_t)len + GSNP_WIN + 512));
@@ -596,7 +594,6 @@ int gsnp_load_reads(gsnp_ctx* c, const gsnp_read_batch* b)
     HIPCHK(hipStreamSynchronize(c->stream));
     c->n_reads = 0;  // set once the uploads below have succeeded
     c->pitch = L;
-    c->buf_gen++;
     c->chrom_id = next_chrom_id();
     c->h_rpos.assign(b->pos, b->pos + b->n);
     HIPCHK(c->rpos.alloc(b->n + 1));
@@ -772,12 +769,8 @@ int gsnp_batched_call(gsnp_ctx* c, uint32_t start, uint32_t n, int emit_text, ui
     if (start % GSNP_WIN) return fail(GSNP_E_ARG, "span must start on a window boundary");
     int rc = c->span_prepare(n);
     if (rc) return rc;
-    const FusedTune& t = c->tune;
-    std::vector<uint64_t> key = {c->buf_gen, c->chrom_id, start, n, (uint64_t)c->p.rank_sum_mode,
-                                 (uint64_t)c->keep_lk, t.min_class};
-    for (int i = 0; i < 6; i++) key.push_back(((uint64_t)t.wpb[i] << 32) | t.max_blocks[i]);
-    rc = c->launch_captured(c->graph_slot(key), key, [&] { c->span_enqueue(start, n); });
-    if (rc) return rc;
+    c->span_enqueue(start, n);
+    HIPCHK(hipGetLastError());
     if (c->p.rank_sum_mode) {
         c->fix_offset = 0;
         rc = c->host_fixups();
@@ -787,7 +780,7 @@ int gsnp_batched_call(gsnp_ctx* c, uint32_t start, uint32_t n, int emit_text, ui
     if (rc) return rc;
     c->ws = start;
     c->built = false;
-    if (emit_text) return c->format_text(0, start, n, start + 1, nbytes, true);
+    if (emit_text) return c->format_text(0, start, n, start + 1, nbytes);
     if (nbytes) *nbytes = 0;
     return GSNP_OK;
 }
@@ -950,14 +943,15 @@ int Ctx::span_prepare(uint32_t n)
     if (head_qs.n < nheads) {
         HIPCHK(hipStreamSynchronize(stream));
         HIPCHK(head_qs.alloc(nheads));
-        buf_gen++;
     }
     return GSNP_OK;
 }
 
 // The device work of one batched span, up to the rank-sum jobs: site matrix,
 // depth classes, fused sort + likelihood + posterior, rank-sum.  Launches
-// only (no copies, no memsets, no host waits), so it can be captured.
+// only (no copies, no host waits), each queued as it is: replayed as captured
+// graphs the same launches took 7 % longer on 100 kb and 5 % on 24 contigs,
+// and a span's first call a quarter longer for the capture.
 void Ctx::span_enqueue(uint32_t start, uint32_t n)
 {
     if (tile_ok) {
@@ -1042,56 +1036,6 @@ void Ctx::span_enqueue_tiles(uint32_t start, uint32_t n)
     }
 }
 
-// Runs enqueue() through a graph captured for `key`, capturing it on first
-// use; eagerly when graphs are off or the stage timers are on (their events
-// belong to the eager stream).  A capture that fails turns graphs off.
-template <class F>
-int Ctx::launch_captured(GraphSlot& slot, const std::vector<uint64_t>& key, F enqueue)
-{
-    if (!use_graphs || timer.on) {
-        enqueue();
-        HIPCHK(hipGetLastError());
-        return GSNP_OK;
-    }
-    if (!slot.exec || slot.key != key) {
-        slot.reset();
-        hipGraph_t g = nullptr;
-        HIPCHK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-        enqueue();
-        hipError_t e = hipStreamEndCapture(stream, &g);
-        if (e == hipSuccess && g) e = hipGraphInstantiate(&slot.exec, g, nullptr, nullptr, 0);
-        if (g) (void)hipGraphDestroy(g);
-        if (e != hipSuccess || !slot.exec) {
-            (void)hipGetLastError();
-            slot.exec = nullptr;
-            use_graphs = false;
-            enqueue();
-            HIPCHK(hipGetLastError());
-            return GSNP_OK;
-        }
-        slot.key = key;
-    }
-    HIPCHK(hipGraphLaunch(slot.exec, stream));
-    return GSNP_OK;
-}
-
-constexpr size_t kMaxGraphs = 256;
-
-// The cached graph for `key`, or an empty slot for it.  Graphs captured
-// before the last buffer (re)allocation are dropped: their pointers are gone.
-GraphSlot& Ctx::graph_slot(const std::vector<uint64_t>& key)
-{
-    if (graphs_gen != buf_gen) {
-        graphs.clear();
-        graphs_gen = buf_gen;
-    }
-    for (auto& g : graphs)
-        if (g->key == key) return *g;
-    if (graphs.size() >= kMaxGraphs) graphs.erase(graphs.begin());
-    graphs.push_back(std::make_unique<GraphSlot>());
-    return *graphs.back();
-}
-
 int Ctx::span_build(uint32_t start, uint32_t n)
 {
     if ((uint64_t)start + n > chr_len) return fail(GSNP_E_ARG, "span outside the chromosome");
@@ -1129,7 +1073,7 @@ static uint64_t text_bound(uint64_t n_sites, size_t name_len) { return n_sites *
 // Formats the rows of sites [offset, offset + n_sites) into `out` (sized by
 // text_bound), or into the context's text buffer when out is null.
 int Ctx::format_text(uint32_t offset, uint32_t ws_abs, uint32_t n_sites, uint32_t pos_base, uint64_t* nbytes,
-                     bool graph, char* out)
+                     char* out)
 {
     const size_t name_len = chr_name.size();
     const uint64_t need = text_bound(n_sites, name_len);
@@ -1137,7 +1081,6 @@ int Ctx::format_text(uint32_t offset, uint32_t ws_abs, uint32_t n_sites, uint32_
         HIPCHK(hipStreamSynchronize(stream));
         HIPCHK(text.alloc(need));
         text_cap = need;
-        buf_gen++;
     }
     char* dst = out ? out : text.p;
     if (gcount.n < 1) HIPCHK(gcount.alloc(1));
@@ -1150,25 +1093,15 @@ int Ctx::format_text(uint32_t offset, uint32_t ws_abs, uint32_t n_sites, uint32_
     SiteArrays a = site_view(offset);
     Results res = result_view(offset);
     const uint32_t nb = (n_sites + kRowBlock - 1) / kRowBlock;
-    auto enqueue = [&] {
-        timer.begin(kStFormat, stream);
-        launch_fill_u32(stream, gcount.p, 1, 0u);
-        launch_rowlen(stream, ref_view(), ws_abs, a, res, n_sites, rc, gidx.p + offset, gtext.p, gcount.p, rowlen.p,
-                      blocksum.p);
-        launch_gtext(stream, a, res, n_sites, gtext.p, gcount.p, rowlen.p, blocksum.p);
-        launch_scan_blocks(stream, blocksum.p, nb, total.p);
-        launch_format(stream, ref_view(), ws_abs, a, res, n_sites, rc, rowlen.p, blocksum.p, dst);
-        timer.end(kStFormat, stream);
-    };
-    if (graph) {
-        const std::vector<uint64_t> key = {buf_gen, chrom_id, 1u, offset, ws_abs, n_sites, pos_base,
-                                           (uint64_t)(uintptr_t)dst};
-        int r = launch_captured(graph_slot(key), key, enqueue);
-        if (r) return r;
-    } else {
-        enqueue();
-        HIPCHK(hipGetLastError());
-    }
+    timer.begin(kStFormat, stream);
+    launch_fill_u32(stream, gcount.p, 1, 0u);
+    launch_rowlen(stream, ref_view(), ws_abs, a, res, n_sites, rc, gidx.p + offset, gtext.p, gcount.p, rowlen.p,
+                  blocksum.p);
+    launch_gtext(stream, a, res, n_sites, gtext.p, gcount.p, rowlen.p, blocksum.p);
+    launch_scan_blocks(stream, blocksum.p, nb, total.p);
+    launch_format(stream, ref_view(), ws_abs, a, res, n_sites, rc, rowlen.p, blocksum.p, dst);
+    timer.end(kStFormat, stream);
+    HIPCHK(hipGetLastError());
     uint64_t t = 0;
     HIPCHK(hipMemcpyAsync(&t, total.p, 8, hipMemcpyDeviceToHost, stream));
     HIPCHK(hipStreamSynchronize(stream));
@@ -1206,16 +1139,15 @@ int Ctx::text_to_host(uint32_t start, uint32_t n, uint64_t* nbytes, const TextSi
     const int i = tp.cur;
     const uint64_t need = text_bound(n, chr_name.size());
     if (tp.dev[i].n < need) {
-        // nothing may still read the old buffer: its copy, or a graph that writes it
+        // nothing queued may still use the old buffer: its copy, or the kernel that writes it
         HIPCHK(hipStreamSynchronize(tp.copy));
         HIPCHK(hipStreamSynchronize(stream));
         HIPCHK(tp.dev[i].alloc(need + need / 8));
-        buf_gen++;
     }
     // the copy of the span formatted into this buffer kBufs spans ago reads it
     if (tp.recorded[i]) HIPCHK(hipStreamWaitEvent(stream, tp.ev_done[i], 0));
     uint64_t len = 0;
-    int rc = format_text(0, start, n, start + 1, &len, true, tp.dev[i].p);
+    int rc = format_text(0, start, n, start + 1, &len, tp.dev[i].p);
     if (rc) return rc;
     if (tp.host_cap[i] < len) {  // that span has been handed on, and its copy has landed
         if (tp.host[i]) HIPCHK(hipHostFree(tp.host[i]));

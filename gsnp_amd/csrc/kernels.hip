@@ -267,8 +267,7 @@ void launch_site_build(hipStream_t st, const ReadView& r, uint64_t r0, uint64_t 
 // order (base, quality descending, cycle, strand) comes out in the first n
 // slots, as kernel/bitonic_kernel.cu:119-176 produces.
 
-// word fill: clears counters and flags with a kernel, so that the sequence
-// can be captured into a graph (memset nodes are avoided there)
+// word fill: clears counters and flags with a kernel (a caller may capture its stream; memset nodes are avoided there)
 __global__ __launch_bounds__(256) void k_fill_u32(uint32_t* p, uint32_t n, uint32_t v)
 {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
