@@ -255,6 +255,7 @@ struct Ctx {
     DevBuf<double> tscore;
     uint32_t qtab_bytes = 0;
     bool tile_ok = false;
+    bool qadj_full = true;
     std::vector<double> h_prank, h_pprior;
     // chromosome (the fields of ChromState; chrom_id names the uploaded
     // inputs, 0: none)

@@ -161,6 +161,7 @@ Tables Ctx::tables() const
     t.qadj = qadj.p;
     t.td = td;
     t.gd = gd;
+    t.qadj_full = qadj_full ? 1 : 0;
     t.lprior = lprior.p;
     t.prank = prank.p;
     t.read_len = p.read_length;
@@ -352,6 +353,7 @@ int create_ctx(const gsnp_params* p, const double* p_matrix, gsnp_ctx** out)
     QadjTable qt = build_qadj_table(p->pcr_dependency, p->global_dependency);
     c->td = qt.td;
     c->gd = qt.gd;
+    c->qadj_full = std::find(qt.v.begin() + (size_t)qt.td * qt.gd, qt.v.end(), 0) == qt.v.end();
     c->h_pprior.resize(128);
     prior_gen(*p, c->h_pprior.data());
     std::vector<double> lp = log_prior_rows(c->h_pprior.data());
@@ -867,9 +869,8 @@ int gsnp_sort_likelihood(gsnp_ctx* c, uint32_t* records, uint32_t pitch, const u
     HIPCHK(hipMemcpyAsync(c->sites.rec.p, rows.data(), rows.size() * 4, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(c->sites.nrec.p, n.data(), 4ull * n_sites, hipMemcpyHostToDevice, c->stream));
     SiteArrays a = c->site_view(0);
-    launch_bucket(c->stream, a.nrec, n_sites, c->lists.p, c->win_cap, c->counts.p, 0, nullptr);
-    launch_sort(c->stream, a.rec, a.nrec, c->lists.p, c->win_cap, c->counts.p, n_sites);
-    launch_likelihood(c->stream, c->tables(), a, n_sites, c->lk.p, c->err.p);
+    launch_sort_likelihood(c->stream, c->tables(), a, n_sites, c->lists.p, c->win_cap, c->counts.p, c->lk.p, c->err.p,
+                           c->tune, nullptr);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(rows.data(), c->sites.rec.p, rows.size() * 4, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipMemcpyAsync(lk10, c->lk.p, 80ull * n_sites, hipMemcpyDeviceToHost, c->stream));

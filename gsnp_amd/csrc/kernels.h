@@ -21,6 +21,7 @@ struct Tables {
     const double* score = nullptr;  // [256*256*4][10]
     const uint8_t* qadj = nullptr;  // [64][td][gd]
     int td = 1, gd = 1;
+    int qadj_full = 1;  // no entry of q in [1,64) is above 255 (0 in the table)
     const double* lprior = nullptr;  // [8][10]
     const double* prank = nullptr;   // 64*64*2048
     int read_len = 100;
@@ -102,6 +103,10 @@ struct FusedArgs {
     uint32_t* err = nullptr;
     int write_lk = 0;   // also store the ten log-likelihoods of each site
     int posterior = 1;  // call the sites (0: likelihoods only, for the per-window path)
+    // caller-owned records (posterior 0): sorted rows written back, and the
+    // sites whose records are not all plain (k_likelihood's sites) listed
+    int store = 0;
+    uint32_t *odd_list = nullptr, *odd_count = nullptr;
 };
 
 // Launch shape of the fused stage: bucket classes below min_class run on
@@ -172,10 +177,15 @@ void launch_site_build(hipStream_t s, const ReadView& r, uint64_t r0, uint64_t r
                        int64_t lo_min, int64_t hi_max, uint32_t carry, const SiteArrays& a, int4* head_qs,
                        uint64_t* range);
 void launch_bucket(hipStream_t s, const int32_t* nrec, uint32_t n_sites, uint32_t* lists, uint32_t list_pitch,
-                   uint32_t* counts, int all, unsigned long long* n_records, int min_class = 0);
+                   uint32_t* counts, int all, unsigned long long* n_records, int min_class = 0,
+                   const uint32_t* skip = nullptr);
 void launch_sort(hipStream_t s, uint32_t* rec, const int32_t* nrec, const uint32_t* lists, uint32_t list_pitch,
                  const uint32_t* counts, uint32_t max_sites);
-void launch_likelihood(hipStream_t s, const Tables& t, const SiteArrays& a, uint32_t n_sites, double* lk, uint32_t* err);
+// sort and likelihood of caller-owned records (rows of 256): counts (8 words)
+// and lists are working memory; nothing happens when *skip (may be null) is set
+void launch_sort_likelihood(hipStream_t s, const Tables& t, const SiteArrays& a, uint32_t n_sites, uint32_t* lists,
+                            uint32_t list_pitch, uint32_t* counts, double* lk, uint32_t* err, const FusedTune& tune,
+                            const uint32_t* skip);
 void launch_posterior(hipStream_t s, const Tables& t, const RefView& ref, uint32_t ws, const SiteArrays& a,
                       uint32_t n_sites, const int4* head_qs, Results& out, RankJob* jobs, uint32_t* job_count);
 void launch_fused(hipStream_t s, const FusedArgs& f, const uint32_t* lists, uint32_t list_pitch, const uint32_t* counts,

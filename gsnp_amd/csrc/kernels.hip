@@ -290,8 +290,9 @@ constexpr uint32_t kBucketPer = 16;
 
 __global__ __launch_bounds__(256) void k_bucket(const int32_t* nrec, uint32_t n_sites, uint32_t* lists,
                                                 uint32_t pitch, uint32_t* counts, int all, int min_class,
-                                                unsigned long long* n_records)
+                                                unsigned long long* n_records, const uint32_t* skip)
 {
+    if (skip && *skip) return;  // the caller's counts are out of range: empty lists
     __shared__ uint32_t cnt[6], base[6];
     __shared__ unsigned long long rsum[4];
     if (threadIdx.x < 6) cnt[threadIdx.x] = 0;
@@ -356,13 +357,13 @@ __global__ __launch_bounds__(256) void k_bucket(const int32_t* nrec, uint32_t n_
 }
 
 void launch_bucket(hipStream_t st, const int32_t* nrec, uint32_t n_sites, uint32_t* lists, uint32_t pitch,
-                   uint32_t* counts, int all, unsigned long long* n_records, int min_class)
+                   uint32_t* counts, int all, unsigned long long* n_records, int min_class, const uint32_t* skip)
 {
     launch_fill_u32(st, counts, 6, 0u);
     const uint32_t blocks = (n_sites + 256 * kBucketPer - 1) / (256 * kBucketPer);
     if (blocks)
         hipLaunchKernelGGL(k_bucket, dim3(blocks), dim3(256), 0, st, nrec, n_sites, lists, pitch, counts, all,
-                           min_class, n_records);
+                           min_class, n_records, skip);
 }
 
 template <int J>
@@ -563,42 +564,40 @@ void launch_sort(hipStream_t st, uint32_t* rec, const int32_t* nrec, const uint3
 }
 
 // ---------------------------------------------------------------------------
-// (c) likelihood.  One thread per site over its sorted records
-// (kernel/likelihood_kernel.cu:168-256): walk_adjusted gives each record's
-// dependency-adjusted quality in record order and the 10 genotype scores of
-// its row (one 128-byte line of the score table) are added in that order.
-__global__ __launch_bounds__(256) void k_likelihood(Tables t, SiteArrays a, uint32_t n_sites, double* lk,
-                                                    uint32_t* err)
+// (c) likelihood of listed sites, one thread per site over its sorted records
+// in memory (kernel/likelihood_kernel.cu:168-256): walk_adjusted gives each
+// record's dependency-adjusted quality in record order and the 10 genotype
+// scores of its row (one 128-byte line of the score table) are added in that
+// order.  It takes the records of a caller that k_fused does not: occurrence
+// bytes other than 1, or bits above the base set.
+__global__ __launch_bounds__(256) void k_likelihood(Tables t, SiteArrays a, const uint32_t* list,
+                                                    const uint32_t* list_count, double* lk, uint32_t* err)
 {
     __shared__ uint32_t seen_all[256 * 17];
     uint32_t* seen = seen_all + threadIdx.x * 17;
-    const uint32_t s = blockIdx.x * 256u + threadIdx.x;
-    if (s >= n_sites) return;
-    const uint32_t n = (uint32_t)a.nrec[s];
-    const uint32_t* row = a.rec + (size_t)s * kSlots;
-    double acc[10];
+    const uint32_t count = *list_count;
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < count; i += gridDim.x * 256u) {
+        const uint32_t s = list[i];
+        const uint32_t n = (uint32_t)a.nrec[s];
+        const uint32_t* row = a.rec + (size_t)s * kSlots;
+        double acc[10];
 #pragma unroll
-    for (int g = 0; g < 10; g++) acc[g] = 0.0;
-    const uint32_t bad = walk_adjusted(row, n, t, seen, [&](uint32_t qa, uint32_t cyc, uint32_t o) {
-        const double2* sr =
-            reinterpret_cast<const double2*>(t.score + (size_t)((qa << 10) | (cyc << 2) | o) * kScoreRowStride);
+        for (int g = 0; g < 10; g++) acc[g] = 0.0;
+        const uint32_t bad = walk_adjusted(row, n, t, seen, [&](uint32_t qa, uint32_t cyc, uint32_t o) {
+            const double2* sr =
+                reinterpret_cast<const double2*>(t.score + (size_t)((qa << 10) | (cyc << 2) | o) * kScoreRowStride);
 #pragma unroll
-        for (int h = 0; h < 5; h++) {
-            const double2 v = sr[h];
-            acc[2 * h] += v.x;
-            acc[2 * h + 1] += v.y;
-        }
-    });
-    double2* out = reinterpret_cast<double2*>(lk + (size_t)s * 10);
+            for (int h = 0; h < 5; h++) {
+                const double2 v = sr[h];
+                acc[2 * h] += v.x;
+                acc[2 * h + 1] += v.y;
+            }
+        });
+        double2* out = reinterpret_cast<double2*>(lk + (size_t)s * 10);
 #pragma unroll
-    for (int h = 0; h < 5; h++) out[h] = make_double2(acc[2 * h], acc[2 * h + 1]);
-    if (bad) atomicOr(err, bad);
-}
-
-void launch_likelihood(hipStream_t st, const Tables& t, const SiteArrays& a, uint32_t n_sites, double* lk, uint32_t* err)
-{
-    const uint32_t blocks = (n_sites + 255) / 256;
-    if (blocks) hipLaunchKernelGGL(k_likelihood, dim3(blocks), dim3(256), 0, st, t, a, n_sites, lk, err);
+        for (int h = 0; h < 5; h++) out[h] = make_double2(acc[2 * h], acc[2 * h + 1]);
+        if (bad) atomicOr(err, bad);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -811,7 +810,10 @@ __host__ __device__ constexpr uint32_t qadj_lds_words(uint32_t td, uint32_t gd)
 // Up to 128 records the kernel is held to 128 VGPRs, four waves per SIMD
 // (the 64-record class would take 148 and three waves; with four, the
 // stage is about 3 % faster); the 256 class keeps its registers.
-template <int S, bool QL = false, bool POST = true>
+// A plain record: one occurrence, nothing above its base.
+__device__ __forceinline__ bool odd_record(uint32_t w) { return (w & 0xFE0000FFu) != 1u; }
+
+template <int S, bool QL = false, bool POST = true, bool STORE = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(S <= 128 ? 4 : 1, 8))) void k_fused(FusedArgs f, const uint32_t* list, const uint32_t* count_ptr)
 {
     constexpr uint32_t G = fused_group<S>();
@@ -888,6 +890,26 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(S <= 128 ? 
                 for (uint32_t k = 0; k < CH; k++) v[k] = e < nk[k] ? v[k] : 0xFFFFFFFFu;
 #pragma unroll
                 for (uint32_t k = 0; k < CH; k += 2) bitonic_all2<2, S>(v[k], v[k + 1], e);  // CH is even
+                if constexpr (STORE) {
+                    uint32_t odd = 0;  // bit k: my record of pass k is not plain
+                    const bool all_odd = !f.t.qadj_full;
+#pragma unroll
+                    for (uint32_t k = 0; k < CH; k++) {
+                        const uint32_t st = (uint32_t)__shfl((int)site, (int)((k0 + k) * P + sub));
+                        if (e < nk[k]) {
+                            f.a.rec[(size_t)st * kSlots + e] = v[k];
+                            odd |= all_odd || odd_record(v[k]) ? 1u << k : 0u;
+                        }
+                    }
+                    if (__ballot(odd != 0)) {
+#pragma unroll 1
+                        for (uint32_t k = 0; k < CH; k++) {
+                            const uint64_t who = __ballot((odd >> k) & 1u) & gmask;
+                            const uint32_t st = (uint32_t)__shfl((int)site, (int)((k0 + k) * P + sub));
+                            if (who && e == 0) f.odd_list[atomicAdd(f.odd_count, 1u)] = st;
+                        }
+                    }
+                }
 #pragma unroll
                 for (uint32_t k = 0; k < CH; k++) {
                     // the lanes of my site that agree with me on every key bit
@@ -950,7 +972,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(S <= 128 ? 
                     srt[((k0 + k) * P + sub) * RS + e] = my ? row : 0u;
                 }
             }
-            if (qf_min == 0u || qa_min == 0u) bad |= kErrQadjRange;
+            // (a table with zeros scores every site of a caller's records in k_likelihood, which sees their own)
+            if (qf_min == 0u || (!STORE && qa_min == 0u)) bad |= kErrQadjRange;
         } else {
             constexpr int R = S / 64;
             uint32_t v[G][R];
@@ -973,12 +996,27 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(S <= 128 ? 
                 for (int r = 0; r < R; r++) bitonic_all<2, 64>(v[gi][r], (uint32_t)(r * 64) + lane);
                 regs_merge<R, 128>(v[gi], lane);
                 if constexpr (S == 256) regs_merge<R, 256>(v[gi], lane);
-                uint32_t slot[R];
+                if constexpr (STORE) {
+                    const uint32_t st = (uint32_t)__builtin_amdgcn_readlane((int)site, (int)gi);
+                    const uint32_t nn = (uint32_t)__builtin_amdgcn_readlane((int)n, (int)gi);
+                    bool odd = false;
+#pragma unroll
+                    for (int r = 0; r < R; r++) {
+                        const uint32_t e = (uint32_t)r * 64u + lane;
+                        if (e < nn) {
+                            f.a.rec[(size_t)st * kSlots + e] = v[gi][r];
+                            odd = odd || !f.t.qadj_full || odd_record(v[gi][r]);
+                        }
+                    }
+                    if (__ballot(odd) && lane == 0) f.odd_list[atomicAdd(f.odd_count, 1u)] = st;
+                }
+                uint32_t slot[R], beyond = 0;
                 wide_slots<R>(v[gi], below, upto, td, gd, bad, slot);
 #pragma unroll
                 for (int r = 0; r < R; r++)  // padding slots: row 0, all +0.0
                     srt[gi * RS + (uint32_t)r * 64u + lane] =
-                        slot[r] != 0xFFFFFFFFu ? score_row(f.t.qadj, slot[r], bad) : 0u;
+                        slot[r] != 0xFFFFFFFFu ? score_row(f.t.qadj, slot[r], beyond) : 0u;
+                if constexpr (!STORE) bad |= beyond;
             }
         }
         wave_lds_sync();
@@ -1056,8 +1094,21 @@ static void launch_fused_class(hipStream_t st, const FusedArgs& f, const uint32_
     uint32_t blocks = (groups + wpb - 1) / wpb;
     if (blocks > max_blocks) blocks = max_blocks;
     if (!blocks) blocks = 1;
-    // the batched form's launches (posterior fused) and the per-window path's
-    // (likelihoods only) are separate instantiations
+    // the calling launches (posterior fused), the per-window path's
+    // (likelihoods only) and those on a caller's records (sorted rows written
+    // back) are separate instantiations
+    if (f.store) {
+        if constexpr (S <= 32) {
+            if (ql) {
+                hipLaunchKernelGGL((k_fused<S, true, false, true>), dim3(blocks), dim3(64 * wpb), table + wpb * per_wave,
+                                   st, f, list, count);
+                return;
+            }
+        }
+        hipLaunchKernelGGL((k_fused<S, false, false, true>), dim3(blocks), dim3(64 * wpb), wpb * per_wave, st, f, list,
+                           count);
+        return;
+    }
     if constexpr (S <= 32) {
         if (ql) {
             if (f.posterior)
@@ -1100,6 +1151,38 @@ void launch_fused(hipStream_t st, const FusedArgs& f, const uint32_t* lists, uin
     // deepest classes first: their groups are the longest
     for (int cls = 5; cls >= (int)tune.min_class; cls--)
         launch_fused_one(st, f, lists, pitch, counts, max_sites, (uint32_t)cls, tune.wpb[cls], tune.max_blocks[cls]);
+}
+
+// The sites go through the same launches as the per-window path's, with the
+// sorted rows written back; those with a record that is not plain are scored
+// again from their sorted rows, one thread each.  200,003 sites of mean depth
+// 30, 1 % of 200-256 records: 3.4 ms with one thread for every site, whose
+// record walk is serial and whose score rows come 16 bytes a lane; 0.25 ms this way.
+void launch_sort_likelihood(hipStream_t st, const Tables& t, const SiteArrays& a, uint32_t n_sites, uint32_t* lists,
+                            uint32_t pitch, uint32_t* counts, double* lk, uint32_t* err, const FusedTune& tune,
+                            const uint32_t* skip)
+{
+    if (!n_sites) return;
+    launch_fill_u32(st, counts + 6, 1, 0u);
+    // class 0 holds no list of its own: the odd sites' place
+    const uint32_t mc = tune.min_class ? tune.min_class : 1u;
+    launch_bucket(st, a.nrec, n_sites, lists, pitch, counts, 1, nullptr, (int)mc, skip);
+    FusedArgs f;
+    f.t = t;
+    f.a = a;
+    f.out.lk = lk;
+    f.err = err;
+    f.write_lk = 1;
+    f.posterior = 0;
+    f.store = 1;
+    f.odd_list = lists;
+    f.odd_count = counts + 6;
+    FusedTune shape = tune;
+    shape.min_class = mc;
+    launch_fused(st, f, lists, pitch, counts, n_sites, shape);
+    const uint32_t blocks = (n_sites + 255) / 256;
+    hipLaunchKernelGGL(k_likelihood, dim3(blocks < 1024u ? blocks : 1024u), dim3(256), 0, st, t, a, f.odd_list,
+                       f.odd_count, lk, err);
 }
 
 void launch_deep_tiles(hipStream_t st, const FusedArgs& f, const ReadView& r, const uint64_t* range, uint32_t n_built,

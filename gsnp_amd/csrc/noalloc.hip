@@ -27,6 +27,7 @@ static __device__ __align__(256) uint32_t scratch[kNoallocWords];
 
 namespace {
 
+constexpr uint32_t kErrCounts = 0x80000000u;  // beside the kernels' flags
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 uint32_t* g_scratch_ptr[kMaxDevices] = {};
@@ -36,7 +37,7 @@ __global__ __launch_bounds__(256) void k_check_counts(const int32_t* counts, uin
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i < n) {
         const int32_t c = counts[i];
-        if (c < 0 || c > (int32_t)kSlots) atomicOr(err, 1u);
+        if (c < 0 || c > (int32_t)kSlots) atomicOr(err, kErrCounts);
     }
 }
 
@@ -86,21 +87,18 @@ extern "C" int gsnp_sort_likelihood_noalloc(gsnp_ctx* c, uint32_t* records, cons
     // class counters are cleared by launch_bucket)
     launch_fill_u32(s, err, 1, 0u);
     hipLaunchKernelGGL(k_check_counts, dim3((n_sites + 255) / 256), dim3(256), 0, s, counts, n_sites, err);
-    uint32_t e = 0;
-    hipError_t he = hipMemcpyAsync(&e, err, 4, hipMemcpyDeviceToHost, s);
-    if (he == hipSuccess) he = hipStreamSynchronize(s);
-    if (he != hipSuccess) return fail(GSNP_E_DEVICE, std::string("count check: ") + hipGetErrorString(he));
-    if (e) return fail(GSNP_E_ARG, "a record count is outside [0, 256]");
     SiteArrays a;
     a.rec = records;
     a.nrec = const_cast<int32_t*>(counts);  // read only on this path
-    launch_bucket(s, a.nrec, n_sites, lists, kNoallocMaxSites, cls_count, 0, nullptr);
-    launch_sort(s, records, a.nrec, lists, kNoallocMaxSites, cls_count, n_sites);
-    launch_likelihood(s, c->tables(), a, n_sites, lk10, err);
-    he = hipGetLastError();
+    // counts out of range leave every list empty, so that nothing of the
+    // caller's is touched; the host sees them with the other errors
+    launch_sort_likelihood(s, c->tables(), a, n_sites, lists, kNoallocMaxSites, cls_count, lk10, err, c->tune, err);
+    uint32_t e = 0;
+    hipError_t he = hipGetLastError();
     if (he == hipSuccess) he = hipMemcpyAsync(&e, err, 4, hipMemcpyDeviceToHost, s);
     if (he == hipSuccess) he = hipStreamSynchronize(s);
     if (he != hipSuccess) return fail(GSNP_E_DEVICE, std::string("sort + likelihood: ") + hipGetErrorString(he));
+    if (e & kErrCounts) return fail(GSNP_E_ARG, "a record count is outside [0, 256]");
     if (e & kErrQadjRange) return fail(GSNP_E_RANGE, "adjusted quality exceeds the score table");
     return GSNP_OK;
 }
