@@ -117,13 +117,6 @@ __device__ __forceinline__ void sort_regs(uint32_t (&v)[D])
     if constexpr (left > m) sort_regs<N, B + m>(v);
 }
 
-__device__ __forceinline__ void lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 __device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 __device__ __forceinline__ uint64_t uniform(uint64_t v)
 {
@@ -390,7 +383,7 @@ __global__ __launch_bounds__(64 * NW) void k_call_tile(TileArgs f, const uint32_
 #pragma unroll
             for (uint32_t c = 0; c < CH; c++)
                 kept_reads[c * 64u + lane] = make_uint2(ms[c] ? (uint32_t)(int32_t)((int64_t)ps[c] - p0) : 0u, ms[c]);
-            lds_sync();
+            wave_lds_sync();
         }
         auto load_read = [&](uint32_t c, int32_t& st, uint32_t& m) {
             if constexpr (CH > 2) {
@@ -420,13 +413,13 @@ __global__ __launch_bounds__(64 * NW) void k_call_tile(TileArgs f, const uint32_
             const uint4 ones = make_uint4(~0u, ~0u, ~0u, ~0u);
 #pragma unroll
             for (uint32_t k = 0; k < kAnchorWords / 256u; k++) z[k * 64u + lane] = ones;
-            lds_sync();
+            wave_lds_sync();
 #pragma unroll 1
             for (uint32_t c = 0; c < nch; c++) {
                 load_read(c, st, m);
                 if (rm_hit(m) == 1) atomicMin(&rec[anchor(st, m)], c * 64u + lane);
             }
-            lds_sync();
+            wave_lds_sync();
 #pragma unroll 1
             for (uint32_t c = 0; c < nch; c++) {
                 load_read(c, st, m);
@@ -438,7 +431,7 @@ __global__ __launch_bounds__(64 * NW) void k_call_tile(TileArgs f, const uint32_
                     }
                 }
             }
-            lds_sync();
+            wave_lds_sync();
 #pragma unroll 1
             for (uint32_t c = 0; c < nch; c++) {
                 load_read(c, st, m);
@@ -461,7 +454,7 @@ __global__ __launch_bounds__(64 * NW) void k_call_tile(TileArgs f, const uint32_
                 n_shared += (uint32_t)__popcll(who);
             }
         }
-        lds_sync();
+        wave_lds_sync();
         {
             uint4* z = reinterpret_cast<uint4*>(mine);
             const uint4 none = make_uint4(kNoRec, kNoRec, kNoRec, kNoRec);
@@ -469,7 +462,7 @@ __global__ __launch_bounds__(64 * NW) void k_call_tile(TileArgs f, const uint32_
             for (uint32_t k = 0; k < (uint32_t)D / 4u; k++) z[k * 64u + lane] = none;
             reinterpret_cast<uint4*>(cnt)[lane] = make_uint4(0, 0, 0, 0);
         }
-        lds_sync();
+        wave_lds_sync();
         uint32_t* slot = rec + lane;  // my next free slot
         int depth = 0, other = 0;     // reads over my site; hit counts of its repeat reads beyond one each
         // my byte of a read of the tile: unconditional (the read store is
@@ -596,11 +589,11 @@ __global__ __launch_bounds__(64 * NW) void k_call_tile(TileArgs f, const uint32_
                     size[l] += (y ^ mem[l]) < 65536u ? 1u : 0u;
                 }
             }
-            lds_sync();
+            wave_lds_sync();
 #pragma unroll
             for (uint32_t l = 0; l < CH; l++)
                 if (l * 64u + lane < n_shared) shared_list[place[l]] = mem[l] | (size[l] > kBigGroup ? 0x80000000u : 0u);
-            lds_sync();
+            wave_lds_sync();
             uint32_t* group = slot;
             uint32_t earlier = 0, id = 0;  // id: 128 + the big group's number, 0 in a small one
 #pragma unroll 1
@@ -642,7 +635,7 @@ __global__ __launch_bounds__(64 * NW) void k_call_tile(TileArgs f, const uint32_
                 }
             }
         }
-        lds_sync();
+        wave_lds_sync();
         const uint32_t n = (uint32_t)(slot - rec) / kTile;  // records of my site
         SiteVals v;
         v.depth = depth;
@@ -657,7 +650,7 @@ __global__ __launch_bounds__(64 * NW) void k_call_tile(TileArgs f, const uint32_
             uint32_t q[D];
 #pragma unroll
             for (int k = 0; k < D; k++) q[k] = rec[k * kTile + lane];
-            lds_sync();  // the parked rows take the columns' place
+            wave_lds_sync();  // the parked rows take the columns' place
             if constexpr (D == 64) {
                 // short spans send every tile up to 64 records here
                 if (M <= 32)
@@ -670,7 +663,7 @@ __global__ __launch_bounds__(64 * NW) void k_call_tile(TileArgs f, const uint32_
             const uint32_t cycles = pitch & 511u;
             if (n_big) {
                 for (uint32_t k = 0; k < n_big; k++) big[k * kTile + lane] = 0;
-                lds_sync();
+                wave_lds_sync();
             }
             uint32_t prev = 0, g = ~0u;  // g: first occurrences of the base so far, minus one
 #pragma unroll
@@ -710,7 +703,7 @@ __global__ __launch_bounds__(64 * NW) void k_call_tile(TileArgs f, const uint32_
                 }
             }
         }
-        lds_sync();
+        wave_lds_sync();
 
         // ---- C: score rows in record order -------------------------------
         const uint64_t nb = uniform(b2), ne = uniform(e2);
@@ -742,14 +735,14 @@ __global__ __launch_bounds__(64 * NW) void k_call_tile(TileArgs f, const uint32_
                     i += 8;
                 }
             }
-            lds_sync();
+            wave_lds_sync();
             if (k) *reinterpret_cast<double2*>(p_at) = make_double2(p_a0, p_a1);
             p_a0 = a0;
             p_a1 = a1;
             p_at = rw + cl;
         }
         *reinterpret_cast<double2*>(p_at) = make_double2(p_a0, p_a1);
-        lds_sync();
+        wave_lds_sync();
 
         // ---- D: call ------------------------------------------------------
         double acc[10];
@@ -771,7 +764,7 @@ __global__ __launch_bounds__(64 * NW) void k_call_tile(TileArgs f, const uint32_
             f.t, f.ref, (uint32_t)p0 + lane, v, [&](int g) { return acc[g]; },
             [&](int g) { return lprior[(ori & 7u) * 10u + (uint32_t)g]; });
         c.called = c.called && in_span;
-        lds_sync();  // the next tile's records take the sums' place
+        wave_lds_sync();  // the next tile's records take the sums' place
         if (in_span) {
             records += n;
             if (f.write_lk) {
@@ -903,7 +896,7 @@ __global__ __launch_bounds__(512) void k_tile_class(ReadView r, uint32_t ws, uin
         if (e - b <= kMaxTileReads) {
             const int64_t p0 = (int64_t)ws + (int64_t)tile * kTile;
             hist[w][lane] = 0;
-            lds_sync();
+            wave_lds_sync();
             auto count = [&](int32_t p, uint32_t m) {
                 const int32_t st = (int32_t)((int64_t)p - p0), en = st + (int32_t)rm_len(m);
                 if (rm_hit(m) == 1 && en > 0) {
@@ -913,7 +906,7 @@ __global__ __launch_bounds__(512) void k_tile_class(ReadView r, uint32_t ws, uin
             };
             count(pos[k], meta[k]);
             for (uint64_t i = b + 64u + lane; i < e; i += 64) count(r.pos[i], r.meta[i]);
-            lds_sync();
+            wave_lds_sync();
             const uint32_t most = wave_max((uint32_t)wave_prefix(hist[w][lane]));
             c = most <= 16 ? 0u : most <= 32 ? 1u : most <= 40 ? 2u : most <= 64 ? 3u : most <= 128 ? 4u : kDeepClass;
             if (e - b > kShallowReads && c < 4u) c = 4u;

@@ -311,16 +311,15 @@ struct Ctx {
     // known SNPs of the chromosome (host copies, for the adjoint's prior rows)
     std::vector<gsnp_snp> h_snps;
     std::vector<uint8_t> h_snp_ref;
-    // adjoint: records of a prepared span in site order, their score-row keys,
-    // their place in key order and the reduction pieces
-    uint32_t adj_start = 0, adj_n = 0, adj_npieces = 0;
+    // adjoint: the record words of a prepared span in site order and sorted by
+    // key within each block of sites, the reduction pieces and the keys in use
+    uint32_t adj_start = 0, adj_n = 0, adj_npieces = 0, adj_nblk = 0, adj_nuk = 0, adj_groups = 0;
     uint64_t adj_nrec = 0;
-    DevBuf<uint32_t> adj_cnt, adj_prow, adj_key, adj_skey, adj_perm, adj_tmp, adj_pstart, adj_kpiece;
-    DevBuf<uint32_t> adj_rsite;  // per record (record order): its site
-    DevBuf<uint32_t> adj_ssite;  // per record in key order: its site
-    DevBuf<uint32_t> adj_hist, adj_mask;
-    DevBuf<uint64_t> adj_off, adj_pidx, adj_hoff, adj_bsum;
-    DevBuf<double> adj_T, adj_w, adj_ll, adj_dh, adj_psum, adj_part, adj_out, adj_pm, adj_grad, adj_lp;
+    DevBuf<uint32_t> adj_cnt, adj_prow, adj_word, adj_sword, adj_tmp, adj_hist, adj_hbase, adj_cbase, adj_cpiece, adj_mask;
+    DevBuf<uint32_t> adj_pstart, adj_pblock, adj_kpiece, adj_used, adj_ukey;
+    DevBuf<uint64_t> adj_off, adj_start_of, adj_pidx, adj_uidx, adj_hoff, adj_bsum;
+    DevBuf<uint2> adj_work;
+    DevBuf<double> adj_T, adj_w, adj_ll, adj_dh, adj_psum, adj_sums, adj_part, adj_out, adj_pm, adj_grad, adj_lp;
     // device dictionary encoder scratch
     DevBuf<int32_t> dict_mm, dict_vals;
     DevBuf<uint32_t> dict_bits, dict_wpre, dict_out;

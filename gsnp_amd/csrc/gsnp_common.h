@@ -10,6 +10,14 @@
 
 namespace gsnp {
 
+// LDS exchange between the lanes of one wave
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Window geometry and limits (cpp/common.h:14-16, :71-81).
 constexpr uint32_t kWin = 262144;     // sites per window (32*8192)
 constexpr uint32_t kSlots = 256;      // record slots per site (MAX_NUM_NON_ZERO)

@@ -88,7 +88,7 @@ struct RowCtx {
 };
 
 // error flags written by kernels
-enum : uint32_t { kErrQadjRange = 1u, kErrRecordOverflow = 2u };
+enum : uint32_t { kErrQadjRange = 1u, kErrRecordOverflow = 2u, kErrAdjQ = 4u /* adjusted quality of 64 or more in the adjoint */ };
 
 // Arguments of the fused sort + likelihood + posterior launch (batched form).
 struct FusedArgs {
@@ -107,6 +107,10 @@ struct FusedArgs {
     // sites whose records are not all plain (k_likelihood's sites) listed
     int store = 0;
     uint32_t *odd_list = nullptr, *odd_count = nullptr;
+    // the adjoint's record words, each site's from key_off on (key_block: a power of two)
+    uint32_t* key_words = nullptr;
+    const uint64_t* key_off = nullptr;
+    uint32_t key_block = 1;
 };
 
 // Launch shape of the fused stage: bucket classes below min_class run on
@@ -179,8 +183,6 @@ void launch_site_build(hipStream_t s, const ReadView& r, uint64_t r0, uint64_t r
 void launch_bucket(hipStream_t s, const int32_t* nrec, uint32_t n_sites, uint32_t* lists, uint32_t list_pitch,
                    uint32_t* counts, int all, unsigned long long* n_records, int min_class = 0,
                    const uint32_t* skip = nullptr);
-void launch_sort(hipStream_t s, uint32_t* rec, const int32_t* nrec, const uint32_t* lists, uint32_t list_pitch,
-                 const uint32_t* counts, uint32_t max_sites);
 // sort and likelihood of caller-owned records (rows of 256): counts (8 words)
 // and lists are working memory; nothing happens when *skip (may be null) is set
 void launch_sort_likelihood(hipStream_t s, const Tables& t, const SiteArrays& a, uint32_t n_sites, uint32_t* lists,

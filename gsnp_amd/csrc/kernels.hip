@@ -5,6 +5,8 @@
 // rounding, so no FMA contraction anywhere.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "gsnp_common.h"
 #include "kernels.h"
 #include "nearest.h"
@@ -258,14 +260,14 @@ void launch_site_build(hipStream_t st, const ReadView& r, uint64_t r0, uint64_t 
 }
 
 // ---------------------------------------------------------------------------
-// (b) segmented sort.  Sites are bucketed by record count (<=8, 16, 32, 64,
-// 128, 256; 0 or 1 record needs no sort) and each bucket runs a bitonic
-// network in registers: for widths up to 64 a site occupies `W` lanes of a
-// wave, exchanging partners with ds_swizzle (xor < 32) or ds_bpermute
-// (xor 32); widths 128/256 keep 2/4 records per lane and do the xor >= 64
-// steps inside the lane.  Padding lanes hold 0xFFFFFFFF, so ascending u32
-// order (base, quality descending, cycle, strand) comes out in the first n
-// slots, as kernel/bitonic_kernel.cu:119-176 produces.
+// (b) sites bucketed by record count (<= 8, 16, 32, 64, 128, 256) and the
+// bitonic networks that the fused launches sort them with, in registers: for
+// widths up to 64 a site occupies as many lanes of a wave, which exchange with
+// ds_swizzle (xor < 32) or ds_bpermute (xor 32); widths 128/256 keep 2/4
+// records per lane and do the xor >= 64 steps inside the lane.  Padding lanes
+// hold 0xFFFFFFFF, so ascending u32 order (base, quality descending, cycle,
+// strand) comes out in the first n slots, as
+// kernel/bitonic_kernel.cu:119-176 produces.
 
 // word fill: clears counters and flags with a kernel (a caller may capture its stream; memset nodes are avoided there)
 __global__ __launch_bounds__(256) void k_fill_u32(uint32_t* p, uint32_t n, uint32_t v)
@@ -448,29 +450,6 @@ __device__ __forceinline__ void bitonic_all2(uint32_t& v0, uint32_t& v1, uint32_
     if constexpr (K < S) bitonic_all2<K * 2, S>(v0, v1, e);
 }
 
-// widths 8..64: 64/S sites per wave, one record per lane
-template <int S>
-__global__ __launch_bounds__(256) void k_sort_lanes(uint32_t* rec, const int32_t* nrec, const uint32_t* list,
-                                                    const uint32_t* count_ptr)
-{
-    const uint32_t count = *count_ptr;
-    const uint32_t lane = lane_id();
-    const uint32_t sub = lane / S, e = lane % S;
-    constexpr uint32_t kPerWave = 64 / S;
-    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const uint32_t nwave = (gridDim.x * blockDim.x) >> 6;
-    for (uint32_t g = wave * kPerWave; g < count; g += nwave * kPerWave) {
-        const uint32_t idx = g + sub;
-        const bool ok = idx < count;
-        uint32_t site = ok ? list[idx] : 0;
-        const uint32_t n = ok ? (uint32_t)nrec[site] : 0;
-        uint32_t* row = rec + (size_t)site * kSlots;
-        uint32_t v = (e < n) ? row[e] : 0xFFFFFFFFu;
-        bitonic_all<2, S>(v, e);
-        if (e < n) row[e] = v;
-    }
-}
-
 // one bitonic merge stage of width K >= 128 over R registers per lane
 // (element e = r*64 + lane): in-lane compare-exchanges for j = K/2 .. 64,
 // then cross-lane j = 32 .. 1; ascending where (e & K) == 0.
@@ -510,57 +489,6 @@ __device__ __forceinline__ void regs_merge(uint32_t* v, uint32_t lane)
 #undef GSNP_XSTEP
         v[r] = x;
     }
-}
-
-// widths 128/256: one site per wave, R = S/64 records per lane at e = r*64+lane
-template <int S>
-__global__ __launch_bounds__(256) void k_sort_regs(uint32_t* rec, const int32_t* nrec, const uint32_t* list,
-                                                   const uint32_t* count_ptr)
-{
-    constexpr int R = S / 64;
-    const uint32_t count = *count_ptr;
-    const uint32_t lane = lane_id();
-    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const uint32_t nwave = (gridDim.x * blockDim.x) >> 6;
-    for (uint32_t g = wave; g < count; g += nwave) {
-        const uint32_t site = list[g];
-        const uint32_t n = (uint32_t)nrec[site];
-        uint32_t* row = rec + (size_t)site * kSlots;
-        uint32_t v[R];
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            const uint32_t e = r * 64 + lane;
-            v[r] = e < n ? row[e] : 0xFFFFFFFFu;
-        }
-        // k = 2..64: every step is cross-lane with e = r*64+lane, (e & k) from lane bits
-#pragma unroll
-        for (int r = 0; r < R; r++) bitonic_all<2, 64>(v[r], (uint32_t)(r * 64) + lane);
-        // k = 128 (and 256): in-lane steps for j >= 64, then cross-lane j = 32..1
-        regs_merge<R, 128>(v, lane);
-        if constexpr (S == 256) regs_merge<R, 256>(v, lane);
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            const uint32_t e = r * 64 + lane;
-            if (e < n) row[e] = v[r];
-        }
-    }
-}
-
-void launch_sort(hipStream_t st, uint32_t* rec, const int32_t* nrec, const uint32_t* lists, uint32_t pitch,
-                 const uint32_t* counts, uint32_t max_sites)
-{
-    if (!max_sites) return;
-    auto grid = [&](uint32_t per_wave) {
-        uint32_t waves = (max_sites + per_wave - 1) / per_wave;
-        uint32_t blocks = (waves + 3) / 4;
-        return blocks < 2048u ? (blocks ? blocks : 1u) : 2048u;
-    };
-    hipLaunchKernelGGL(k_sort_lanes<8>, dim3(grid(8)), dim3(256), 0, st, rec, nrec, lists + 0 * (size_t)pitch, counts + 0);
-    hipLaunchKernelGGL(k_sort_lanes<16>, dim3(grid(4)), dim3(256), 0, st, rec, nrec, lists + 1 * (size_t)pitch, counts + 1);
-    hipLaunchKernelGGL(k_sort_lanes<32>, dim3(grid(2)), dim3(256), 0, st, rec, nrec, lists + 2 * (size_t)pitch, counts + 2);
-    hipLaunchKernelGGL(k_sort_lanes<64>, dim3(grid(1)), dim3(256), 0, st, rec, nrec, lists + 3 * (size_t)pitch, counts + 3);
-    hipLaunchKernelGGL(k_sort_regs<128>, dim3(grid(1)), dim3(256), 0, st, rec, nrec, lists + 4 * (size_t)pitch, counts + 4);
-    hipLaunchKernelGGL(k_sort_regs<256>, dim3(grid(1)), dim3(256), 0, st, rec, nrec, lists + 5 * (size_t)pitch, counts + 5);
 }
 
 // ---------------------------------------------------------------------------
@@ -656,7 +584,7 @@ void launch_posterior(hipStream_t st, const Tables& t, const RefView& ref, uint3
 // lane i owns site i of the group.
 //  1. Sort: the record slots of a chunk of passes are loaded first (the loads
 //     are in flight together), then for S <= 64 lane groups of S sort 64/S
-//     sites per pass with the k_sort_lanes networks, for S = 128/256 one site
+//     sites per pass with the networks above, for S = 128/256 one site
 //     per pass with S/64 records per lane.  Each sorted record then learns,
 //     in parallel (kernel/likelihood_kernel.cu:168-256 walks them in order):
 //       t - 1: how many records before it share its (base, strand, cycle)
@@ -695,13 +623,6 @@ template <int S>
 constexpr uint32_t fused_row_stride()
 {
     return S + 1 < 21 ? 21u : (uint32_t)S + 1u;
-}
-
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // (q, t - 1, g) table index << 10 | cycle << 2 | base of a sorted record
@@ -810,12 +731,28 @@ __host__ __device__ constexpr uint32_t qadj_lds_words(uint32_t td, uint32_t gd)
 // Up to 128 records the kernel is held to 128 VGPRs, four waves per SIMD
 // (the 64-record class would take 148 and three waves; with four, the
 // stage is about 3 % faster); the 256 class keeps its registers.
+// The adjoint's word of a record: its score row (16 bits for an adjusted
+// quality below 64, the gradient table's) and its site within a block of sites.
+__device__ __forceinline__ uint32_t key_word(uint32_t row, uint32_t site, uint32_t block, uint32_t& bad)
+{
+    if (row >= 1u << 16) {
+        bad |= kErrAdjQ;
+        row = (63u << 10) | (row & 1023u);
+    }
+    return (row << 16) | (site & (block - 1u));
+}
+
 // A plain record: one occurrence, nothing above its base.
 __device__ __forceinline__ bool odd_record(uint32_t w) { return (w & 0xFE0000FFu) != 1u; }
 
-template <int S, bool QL = false, bool POST = true, bool STORE = false>
+// What a launch leaves of its sites: calls, log-likelihoods, log-likelihoods
+// and the sorted rows, or the adjoint's record words.
+enum FusedMode : int { kFusedCall = 0, kFusedScore, kFusedStore, kFusedKeys };
+
+template <int S, bool QL, int MODE>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(S <= 128 ? 4 : 1, 8))) void k_fused(FusedArgs f, const uint32_t* list, const uint32_t* count_ptr)
 {
+    constexpr bool POST = MODE == kFusedCall, STORE = MODE == kFusedStore, KEYS = MODE == kFusedKeys;
     constexpr uint32_t G = fused_group<S>();
     constexpr uint32_t RS = fused_row_stride<S>();
     extern __shared__ uint32_t lds[];
@@ -851,7 +788,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(S <= 128 ? 
         // lane gi owns site gi of the group
         const bool act = lane < gcount;
         const uint32_t site = act ? list[g0 + lane] : 0u;
-        const uint32_t n = act ? (uint32_t)f.a.nrec[site] : 0u;
+        const uint64_t key0 = KEYS && act ? f.key_off[site] : 0ull;
+        // (a site that is not called has no words)
+        const uint32_t n = !act ? 0u : KEYS ? (uint32_t)(f.key_off[site + 1] - key0) : (uint32_t)f.a.nrec[site];
         wave_lds_sync();  // the previous group's rows have been read
         // phase 1: sort, dependency counts, score rows parked in LDS
         if constexpr (S <= 64) {
@@ -969,7 +908,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(S <= 128 ? 
                     const uint32_t qa = qtab[v[k] >> 10];  // 0 marks a quality beyond the table
                     qa_min = my && qa < qa_min ? qa : qa_min;
                     const uint32_t row = ((qa > 1u ? qa : 1u) << 10) | (v[k] & 1023u);
-                    srt[((k0 + k) * P + sub) * RS + e] = my ? row : 0u;
+                    if constexpr (KEYS) {
+                        const uint32_t gi = (k0 + k) * P + sub;
+                        const uint32_t st = (uint32_t)__shfl((int)site, (int)gi);
+                        const uint64_t at = ((uint64_t)(uint32_t)__shfl((int)(uint32_t)(key0 >> 32), (int)gi) << 32) |
+                                            (uint32_t)__shfl((int)(uint32_t)key0, (int)gi);
+                        if (my) f.key_words[at + e] = key_word(row, st, f.key_block, bad);
+                    } else {
+                        srt[((k0 + k) * P + sub) * RS + e] = my ? row : 0u;
+                    }
                 }
             }
             // (a table with zeros scores every site of a caller's records in k_likelihood, which sees their own)
@@ -1012,6 +959,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(S <= 128 ? 
                 }
                 uint32_t slot[R], beyond = 0;
                 wide_slots<R>(v[gi], below, upto, td, gd, bad, slot);
+                if constexpr (KEYS) {
+                    const uint32_t st = (uint32_t)__builtin_amdgcn_readlane((int)site, (int)gi);
+                    const uint64_t at =
+                        ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(key0 >> 32), (int)gi) << 32) |
+                        (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)key0, (int)gi);
+#pragma unroll
+                    for (int r = 0; r < R; r++)
+                        if (slot[r] != 0xFFFFFFFFu)
+                            f.key_words[at + (uint32_t)r * 64u + lane] =
+                                key_word(score_row(f.t.qadj, slot[r], bad), st, f.key_block, bad);
+                    continue;
+                }
 #pragma unroll
                 for (int r = 0; r < R; r++)  // padding slots: row 0, all +0.0
                     srt[gi * RS + (uint32_t)r * 64u + lane] =
@@ -1019,6 +978,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(S <= 128 ? 
                 if constexpr (!STORE) bad |= beyond;
             }
         }
+        if constexpr (KEYS) continue;
         wave_lds_sync();
         // phase 2: twelve sites at a time, lane (sl, cl) adds genotypes 2cl and
         // 2cl+1 of site r * 12 + sl in record order, eight records in flight; the
@@ -1094,37 +1054,27 @@ static void launch_fused_class(hipStream_t st, const FusedArgs& f, const uint32_
     uint32_t blocks = (groups + wpb - 1) / wpb;
     if (blocks > max_blocks) blocks = max_blocks;
     if (!blocks) blocks = 1;
-    // the calling launches (posterior fused), the per-window path's
-    // (likelihoods only) and those on a caller's records (sorted rows written
-    // back) are separate instantiations
-    if (f.store) {
+    const uint32_t lds = table + wpb * per_wave;
+    // the calling launches, the per-window path's, those on a caller's records
+    // and the adjoint's are separate instantiations
+    auto launch = [&](auto mode) {
+        constexpr int M = decltype(mode)::value;
         if constexpr (S <= 32) {
             if (ql) {
-                hipLaunchKernelGGL((k_fused<S, true, false, true>), dim3(blocks), dim3(64 * wpb), table + wpb * per_wave,
-                                   st, f, list, count);
+                hipLaunchKernelGGL((k_fused<S, true, M>), dim3(blocks), dim3(64 * wpb), lds, st, f, list, count);
                 return;
             }
         }
-        hipLaunchKernelGGL((k_fused<S, false, false, true>), dim3(blocks), dim3(64 * wpb), wpb * per_wave, st, f, list,
-                           count);
-        return;
-    }
-    if constexpr (S <= 32) {
-        if (ql) {
-            if (f.posterior)
-                hipLaunchKernelGGL((k_fused<S, true, true>), dim3(blocks), dim3(64 * wpb), table + wpb * per_wave, st,
-                                   f, list, count);
-            else
-                hipLaunchKernelGGL((k_fused<S, true, false>), dim3(blocks), dim3(64 * wpb), table + wpb * per_wave, st,
-                                   f, list, count);
-            return;
-        }
-    }
-    if (f.posterior)
-        hipLaunchKernelGGL((k_fused<S, false, true>), dim3(blocks), dim3(64 * wpb), wpb * per_wave, st, f, list, count);
+        hipLaunchKernelGGL((k_fused<S, false, M>), dim3(blocks), dim3(64 * wpb), lds, st, f, list, count);
+    };
+    if (f.key_words)
+        launch(std::integral_constant<int, kFusedKeys>());
+    else if (f.store)
+        launch(std::integral_constant<int, kFusedStore>());
+    else if (f.posterior)
+        launch(std::integral_constant<int, kFusedCall>());
     else
-        hipLaunchKernelGGL((k_fused<S, false, false>), dim3(blocks), dim3(64 * wpb), wpb * per_wave, st, f, list,
-                           count);
+        launch(std::integral_constant<int, kFusedScore>());
 }
 
 void launch_fused_one(hipStream_t st, const FusedArgs& f, const uint32_t* lists, uint32_t pitch,

@@ -1,0 +1,105 @@
+"""The adjoint's records and gradient at the edges of its blocks of 16,384
+sites, reduction chunks of 64 records and depth classes (1 to 255 records a
+site): keys against the calling path's log-likelihoods and against the whole
+span's, the gradient against torch autograd in 64 bits."""
+from __future__ import annotations
+
+import ctypes
+import math
+import random
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+L = 50
+BLOCK, CHUNK = 16384, 64
+DEPTHS = [1, 2, 7, 8, 9, 16, 17, 32, 33, 64, 65, 128, 129, 200, 400]
+
+
+@pytest.fixture(scope="module")
+def spans(built, tmp_path_factory):
+    import gsnp_amd
+    from gsnp_amd.adjoint import Adjoint
+
+    root = tmp_path_factory.mktemp("spans")
+    rng = random.Random(5)
+    n = 2 * BLOCK + 700
+    seq = "".join(rng.choices("ACGT", k=n))
+    seq = seq[:900] + "N" * 150 + seq[1050:]
+    starts = [p for p in range(0, n - L, 4)]  # about twelve reads over a site
+    starts = [p for p in starts if not 700 <= p < 1200]
+    for i, d in enumerate(DEPTHS):  # d - 12 more over a stretch, at either side of the blocks' bound
+        for at in (2000 + 200 * i, BLOCK - 60 + 3 * i):
+            starts += [at + k % 7 for k in range(max(0, d - 12))]
+    starts += [1040 + 5 * k for k in range(3)]  # single records, some over the N run
+    starts.sort()
+    lines = []
+    for i, p in enumerate(starts):
+        ref = seq[p:p + L]
+        s = "".join(rng.choice("AG") if b == "N" else b if rng.random() >= 0.03 else rng.choice("ACGTN") for b in ref)
+        q = "".join(chr(64 + rng.choice([30, 30, 30, 40, rng.randint(1, 45)])) for _ in s)
+        lines.append(f"r{i}\t{s}\t{q}\t{rng.choice([1, 1, 1, 2])}\ta\t{L}\t{rng.choice('+-')}\tc\t{p + 1}\t0\n")
+    fa, so = root / "g.fa", root / "d.soap"
+    fa.write_text(">c\n" + "\n".join(seq[i:i + 60] for i in range(0, n, 60)) + "\n")
+    so.write_text("".join(lines))
+    p0 = gsnp_amd.matrix_gen(fa, so, read_length=L)
+    job = gsnp_amd.Job(fa, so, read_length=L)
+    adj = Adjoint(job)
+    yield job, n, p0, adj.export()
+    job.close()
+
+
+def test_keys_give_the_calling_likelihoods(spans):
+    import gsnp_amd
+
+    job, n, p0, (keys, off, prow) = spans
+    depth = np.diff(off)
+    assert {1, 255} <= set(depth.tolist()) and np.all(depth[prow == 0xFFFFFFFF] == 0)
+    block = np.repeat(np.arange(n) // BLOCK, depth.astype(np.int64))
+    assert np.unique(block << np.int64(16) | keys, return_counts=True)[1].max() > CHUNK
+    job.call(batched=0, emit_text=False)
+    lk = np.zeros((n, 10))
+    out = gsnp_amd.WindowOut()
+    out.lk10 = lk.ctypes.data
+    gsnp_amd.check(gsnp_amd.lib().gsnp_window_results(job.ctx, n, ctypes.byref(out)))
+    p = p0.reshape(256, 256, 4, 4)[:64].transpose(0, 1, 3, 2).reshape(-1, 4)  # [key][allele]
+    rows = np.stack([np.log10(0.5 * p[:, a] + 0.5 * p[:, b]) for a in range(4) for b in range(a, 4)], axis=1)
+    mine = np.zeros((n, 10))
+    np.add.at(mine, np.repeat(np.arange(n), depth.astype(np.int64)), rows[keys])
+    called = prow != 0xFFFFFFFF
+    # at most 255 terms: 255 * 2^-53 relative to the sum of their sizes, all of one sign up to rounding
+    assert np.allclose(mine[called], lk[called], rtol=1e-12, atol=1e-12)
+
+
+@pytest.mark.parametrize("start,size", [(0, 1), (1039, 2), (0, BLOCK - 1), (0, BLOCK), (0, BLOCK + 1), (900, 150),
+                                        (17, 2 * BLOCK), (2000, 3200), (0, 2 * BLOCK + 700)])
+def test_span_edges_match_autograd(spans, start, size):
+    import torch
+
+    from gsnp_amd.adjoint import Adjoint, reference_loglik_torch
+
+    job, n, p0, (keys, off, prow) = spans
+    lh = math.log(job._p.het_novel_r)
+    adj = Adjoint(job, 0, start, size)
+    ll, grad, dh = adj.eval(p0, lh)
+    k, o, r = adj.export()
+    assert np.array_equal(k, keys[int(off[start]):int(off[start + size])])
+    assert np.array_equal(o, off[start:start + size + 1] - off[start]) and np.array_equal(r, prow[start:start + size])
+    if not k.size:
+        assert np.all(grad == 0.0)
+        return
+    lp, mask = adj.priors(lh)
+    log_p = torch.tensor(np.log(p0.reshape(256, 256, 4, 4)[:64]), dtype=torch.float64, requires_grad=True)
+    log_het = torch.tensor(lh, dtype=torch.float64, requires_grad=True)
+    ref = reference_loglik_torch(log_p, log_het, k, o, r, lp, mask, lh)
+    ref.backward()
+    assert abs(float(ref.detach()) - ll) <= 1e-11 * abs(ll) + 1e-13
+    g = log_p.grad.numpy()
+    assert np.allclose(grad, g, rtol=1e-9, atol=1e-12 * np.abs(g).max())
+    unused = np.setdiff1d(np.arange(65536), k)
+    assert np.all(grad.transpose(0, 1, 3, 2).reshape(-1, 4)[unused] == 0.0)
+    assert abs(float(log_het.grad) - dh) <= 1e-9 * abs(dh) + 1e-13
+    again = adj.eval(p0, lh)
+    assert np.array_equal(again[1].view(np.uint64), grad.view(np.uint64))
