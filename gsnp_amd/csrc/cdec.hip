@@ -10,13 +10,17 @@
 // scattered -- then sizes and writes every row.
 #include <hip/hip_runtime.h>
 
+#include <fcntl.h>
+#include <unistd.h>
+
 #include <algorithm>
+#include <cerrno>
 #include <cmath>
-#include <cstdio>
 #include <cstring>
-#include <memory>
+#include <future>
 #include <string>
 #include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "../../include/gsnp_abi.h"
@@ -169,18 +173,25 @@ __global__ __launch_bounds__(256) void k_dec_unpack(const uint8_t* blob, int32_t
     }
 }
 
-// run lengths -> exclusive run starts, one workgroup per column of a window
-__global__ __launch_bounds__(256) void k_dec_starts(int32_t* scratch32, const Expand* items)
+// run lengths -> exclusive run starts, one workgroup per column of a window.
+// Bound by the chain of tiles: 4,096 lengths a tile instead of 256 (8 windows of
+// 262,144 sites, 48 columns: 135 us, was 635).
+__global__ __launch_bounds__(1024) void k_dec_starts(int32_t* scratch32, const Expand* items)
 {
-    __shared__ uint32_t wsum[4];
+    __shared__ uint32_t wsum[16];
     const Expand& x = items[blockIdx.x];
     uint32_t* v = reinterpret_cast<uint32_t*>(scratch32) + x.starts;
-    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6, nrun = x.nrun;
     uint32_t carry = 0;
-    for (uint32_t base = 0; base < x.nrun; base += 256u) {
-        const uint32_t i = base + threadIdx.x;
-        const uint32_t len = i < x.nrun ? v[i] : 0u;
-        uint32_t incl = len;
+    for (uint32_t base = 0; base < nrun; base += 4096u) {
+        const uint32_t i = base + threadIdx.x * 4u;
+        uint32_t len[4], sum = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++) {
+            len[k] = i + k < nrun ? v[i + k] : 0u;
+            sum += len[k];
+        }
+        uint32_t incl = sum;
         for (int off = 1; off < 64; off <<= 1) {
             const uint32_t y = __shfl_up(incl, off);
             if ((int)lane >= off) incl += y;
@@ -188,11 +199,16 @@ __global__ __launch_bounds__(256) void k_dec_starts(int32_t* scratch32, const Ex
         if (lane == 63) wsum[w] = incl;
         __syncthreads();
         uint32_t before = 0, tile = 0;
-        for (uint32_t k = 0; k < 4; k++) {
+        for (uint32_t k = 0; k < 16; k++) {
             if (k < w) before += wsum[k];
             tile += wsum[k];
         }
-        if (i < x.nrun) v[i] = carry + before + incl - len;
+        uint32_t at = carry + before + incl - sum;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++) {
+            if (i + k < nrun) v[i + k] = at;
+            at += len[k];
+        }
         carry += tile;
         __syncthreads();
     }
@@ -504,118 +520,193 @@ std::vector<uint64_t> prefix_of(const std::vector<T>& items)
     return pre;
 }
 
-struct DevMem {
-    std::vector<void*> ptrs;
-    ~DevMem()
+// The output file, opened (and, where it exists, emptied) while the first
+// windows are read: giving back 120 MB of cached pages takes 16 ms.
+struct OutFile {
+    int fd = -1;
+    std::future<int> opening;
+    explicit OutFile(const std::string& out)
+        : opening(std::async([out] { return ::open(out.c_str(), O_WRONLY | O_CREAT | O_TRUNC | O_CLOEXEC, 0666); }))
     {
-        for (void* p : ptrs) (void)hipFree(p);
     }
-    template <class T>
-    hipError_t alloc(T** p, size_t count)
+    OutFile(const OutFile&) = delete;
+    ~OutFile() { close(); }
+    bool ready()
     {
-        void* v = nullptr;
-        hipError_t e = hipMalloc(&v, std::max<size_t>(1, count) * sizeof(T));
-        if (e == hipSuccess) ptrs.push_back(v);
-        *p = static_cast<T*>(v);
-        return e;
+        if (opening.valid()) fd = opening.get();
+        return fd >= 0;
+    }
+    bool write(const char* p, size_t n)
+    {
+        while (n) {
+            const ssize_t k = ::write(fd, p, n);
+            if (k < 0 && errno == EINTR) continue;
+            if (k <= 0) return false;
+            p += k;
+            n -= (size_t)k;
+        }
+        return true;
+    }
+    bool close()
+    {
+        if (!ready()) return false;
+        const int f = fd;
+        fd = -1;
+        return ::close(f) == 0;
     }
 };
 
-// The device work of one batch; the rows go to fo.
-int decode_batch(hipStream_t st, Batch& b, FILE* fo, const std::string& out)
+// What the batches of one call share: a stream, the device memory (kept
+// between batches) and two pinned pieces for the text on its way to the file.
+constexpr size_t kPieceBytes = 2u << 20;
+
+struct Decoder {
+    hipStream_t st = nullptr;
+    DevBuf<uint8_t> mem;
+    DevBuf<char> text;
+    char* piece[2] = {nullptr, nullptr};
+    hipEvent_t ev[2] = {nullptr, nullptr};
+    std::future<std::pair<int, std::string>> drain;  // the last batch's text, on its way; its failure
+    Decoder() = default;
+    Decoder(const Decoder&) = delete;
+    ~Decoder()
+    {
+        if (drain.valid()) drain.wait();
+        if (st) (void)hipStreamSynchronize(st);
+        for (int k = 0; k < 2; k++) {
+            if (ev[k]) (void)hipEventDestroy(ev[k]);
+            if (piece[k]) (void)hipHostFree(piece[k]);
+        }
+        if (st) (void)hipStreamDestroy(st);
+    }
+    hipError_t init()
+    {
+        hipError_t e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
+        for (int k = 0; k < 2 && e == hipSuccess; k++) {
+            e = hipHostMalloc(reinterpret_cast<void**>(&piece[k]), kPieceBytes, hipHostMallocDefault);
+            if (e == hipSuccess) e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
+        }
+        return e;
+    }
+    int finish()
+    {
+        if (!drain.valid()) return GSNP_OK;
+        const auto r = drain.get();
+        return r.first ? fail(r.first, r.second) : GSNP_OK;
+    }
+};
+
+// The text to the file, piece by piece: a piece is written while the next one
+// is copied.  (One pageable copy of the whole text, then one write, took 28 ms
+// for 121 MB before the 12 ms of the write, and 5 ms to give the buffer back.)
+std::pair<int, std::string> write_text(Decoder& d, int device, uint64_t bytes, OutFile& fo, const std::string& out)
 {
-    if (!b.sites) return GSNP_OK;
-    DevMem m;
-    uint8_t* blob;
+    hipError_t e = hipSetDevice(device);
+    if (!fo.ready()) return {GSNP_E_IO, "cannot create " + out};
+    auto size = [&](uint64_t at) { return (size_t)std::min<uint64_t>(kPieceBytes, bytes - at); };
+    auto fetch = [&](uint64_t at, int k) {
+        if (e == hipSuccess) e = hipMemcpyAsync(d.piece[k], d.text.p + at, size(at), hipMemcpyDeviceToHost, d.st);
+        if (e == hipSuccess) e = hipEventRecord(d.ev[k], d.st);
+    };
+    if (bytes) fetch(0, 0);
+    int k = 0;
+    bool ok = true;
+    for (uint64_t at = 0; at < bytes && ok && e == hipSuccess; at += kPieceBytes, k ^= 1) {
+        if (at + kPieceBytes < bytes) fetch(at + kPieceBytes, k ^ 1);
+        if (e == hipSuccess) e = hipEventSynchronize(d.ev[k]);
+        if (e == hipSuccess) ok = fo.write(d.piece[k], size(at));
+    }
+    if (e != hipSuccess) return {GSNP_E_DEVICE, std::string("text copy: ") + hipGetErrorString(e)};
+    if (!ok) return {GSNP_E_IO, "cannot write " + out};
+    return {GSNP_OK, std::string()};
+}
+
+// The device work of one batch; the rows go to fo while the caller reads on.
+int decode_batch(Decoder& d, Batch& b, OutFile& fo, const std::string& out)
+{
+    int rc = d.finish();  // the last batch's text is out of the way
+    if (rc || !b.sites) return rc;
+    hipStream_t st = d.st;
+    const uint64_t n = b.sites, nblk = (n + 255) / 256;
+    // item lists and their element prefixes travel with the blob
+    struct List {
+        uint64_t items, pre, total;
+        uint32_t n;
+    };
+    auto list = [&](const auto& items) {
+        const std::vector<uint64_t> pre = prefix_of(items);
+        return List{b.put(items), b.put(pre), pre.back(), (uint32_t)items.size()};
+    };
+    const List tb = list(b.twobit), s1 = list(b.scat1), s2 = list(b.scat2), s3 = list(b.scat3), up = list(b.unpack),
+               ex = list(b.expand);
+    const uint64_t wins_at = b.put(b.wins);
+    // one allocation: sizes first, then the pointers
     DecCols c;
-    DECCHK(m.alloc(&blob, b.blob.size()));
-    DECCHK(hipMemcpyAsync(blob, b.blob.data(), b.blob.size(), hipMemcpyHostToDevice, st));
-    const uint64_t n = b.sites;
-    DECCHK(m.alloc(&c.c3, n));
-    DECCHK(m.alloc(&c.c4, n));
-    DECCHK(m.alloc(&c.c6, n));
-    DECCHK(m.alloc(&c.c10, n));
-    for (int32_t** p : {&c.c5, &c.c7, &c.c8, &c.c9, &c.c11, &c.c12, &c.c13, &c.c14, &c.c17}) DECCHK(m.alloc(p, n));
-    DECCHK(m.alloc(&c.c15, n));
-    DECCHK(m.alloc(&c.c16, n));
+    uint8_t* blob;
     int32_t* s32;
     double* s64;
-    DECCHK(m.alloc(&s32, b.n32));
-    DECCHK(m.alloc(&s64, b.n64));
-    // item lists and their element prefixes
-    auto upload = [&](const auto& items, auto** d_items, uint64_t** d_pre) -> int {
-        using T = typename std::decay_t<decltype(items)>::value_type;
-        const std::vector<uint64_t> pre = prefix_of(items);
-        DECCHK(m.alloc(d_items, items.size()));
-        DECCHK(m.alloc(d_pre, pre.size()));
-        if (!items.empty()) DECCHK(hipMemcpyAsync(*d_items, items.data(), items.size() * sizeof(T), hipMemcpyHostToDevice, st));
-        DECCHK(hipMemcpyAsync(*d_pre, pre.data(), pre.size() * 8, hipMemcpyHostToDevice, st));
-        return GSNP_OK;
-    };
-    TwoBit* d_tb;
-    Scatter *d_s1, *d_s2, *d_s3;
-    Unpack* d_up;
-    Expand* d_ex;
-    uint64_t *p_tb, *p_s1, *p_s2, *p_s3, *p_up, *p_ex;
-    int rc = upload(b.twobit, &d_tb, &p_tb);
-    if (!rc) rc = upload(b.scat1, &d_s1, &p_s1);
-    if (!rc) rc = upload(b.scat2, &d_s2, &p_s2);
-    if (!rc) rc = upload(b.scat3, &d_s3, &p_s3);
-    if (!rc) rc = upload(b.unpack, &d_up, &p_up);
-    if (!rc) rc = upload(b.expand, &d_ex, &p_ex);
-    if (rc) return rc;
-    auto total = [](const auto& items) {
-        uint64_t t = 0;
-        for (const auto& x : items) t += x.n;
-        return t;
-    };
-    hipLaunchKernelGGL(k_dec_init, dim3(grid_for(n)), dim3(256), 0, st, c, n);
-    if (!b.twobit.empty())
-        hipLaunchKernelGGL(k_dec_2bit, dim3(grid_for(total(b.twobit))), dim3(256), 0, st, c, blob, d_tb, p_tb,
-                           (uint32_t)b.twobit.size());
-    if (!b.scat1.empty())
-        hipLaunchKernelGGL(k_dec_scatter, dim3(grid_for(total(b.scat1))), dim3(256), 0, st, c, blob, s32, d_s1, p_s1,
-                           (uint32_t)b.scat1.size());
-    hipLaunchKernelGGL(k_dec_copy3, dim3(grid_for(n)), dim3(256), 0, st, c, n);
-    if (!b.unpack.empty())
-        hipLaunchKernelGGL(k_dec_unpack, dim3(grid_for(total(b.unpack))), dim3(256), 0, st, blob, s32, s64, d_up, p_up,
-                           (uint32_t)b.unpack.size());
-    if (!b.scat2.empty())
-        hipLaunchKernelGGL(k_dec_scatter, dim3(grid_for(total(b.scat2))), dim3(256), 0, st, c, blob, s32, d_s2, p_s2,
-                           (uint32_t)b.scat2.size());
-    if (!b.scat3.empty())
-        hipLaunchKernelGGL(k_dec_scatter, dim3(grid_for(total(b.scat3))), dim3(256), 0, st, c, blob, s32, d_s3, p_s3,
-                           (uint32_t)b.scat3.size());
-    if (!b.expand.empty()) {
-        hipLaunchKernelGGL(k_dec_starts, dim3((uint32_t)b.expand.size()), dim3(256), 0, st, s32, d_ex);
-        hipLaunchKernelGGL(k_dec_expand, dim3(grid_for(total(b.expand))), dim3(256), 0, st, c, s32, s64, d_ex, p_ex,
-                           (uint32_t)b.expand.size());
-    }
-    // rows: lengths, block offsets, text
-    DecWin* d_w;
-    DECCHK(m.alloc(&d_w, b.wins.size()));
-    DECCHK(hipMemcpyAsync(d_w, b.wins.data(), b.wins.size() * sizeof(DecWin), hipMemcpyHostToDevice, st));
-    const uint64_t nblk = (n + 255) / 256;
     uint32_t* rowlen;
     uint64_t *bsum, *tot;
-    DECCHK(m.alloc(&rowlen, n));
-    DECCHK(m.alloc(&bsum, nblk));
-    DECCHK(m.alloc(&tot, 1));
-    hipLaunchKernelGGL(k_dec_rowlen, dim3((uint32_t)nblk), dim3(256), 0, st, c, blob, d_w, (uint32_t)b.wins.size(), n,
+    size_t used = 0;
+    auto lay = [&](uint8_t* base) {
+        used = 0;
+        auto take = [&](auto** p, uint64_t count) {
+            using T = std::remove_pointer_t<std::remove_pointer_t<decltype(p)>>;
+            *p = base ? reinterpret_cast<T*>(base + used) : nullptr;
+            used = (used + count * sizeof(T) + 255) & ~size_t(255);
+        };
+        take(&blob, b.blob.size());
+        for (char** p : {&c.c3, &c.c4, &c.c6, &c.c10}) take(p, n);
+        for (int32_t** p : {&c.c5, &c.c7, &c.c8, &c.c9, &c.c11, &c.c12, &c.c13, &c.c14, &c.c17}) take(p, n);
+        take(&c.c15, n);
+        take(&c.c16, n);
+        take(&s32, b.n32);
+        take(&s64, b.n64);
+        take(&rowlen, n);
+        take(&bsum, nblk);
+        take(&tot, 1);
+    };
+    lay(nullptr);
+    if (d.mem.n < used) DECCHK(d.mem.alloc(used));
+    lay(d.mem.p);
+    DECCHK(hipMemcpyAsync(blob, b.blob.data(), b.blob.size(), hipMemcpyHostToDevice, st));
+    auto pre = [&](const List& l) { return reinterpret_cast<const uint64_t*>(blob + l.pre); };
+    hipLaunchKernelGGL(k_dec_init, dim3(grid_for(n)), dim3(256), 0, st, c, n);
+    if (tb.n)
+        hipLaunchKernelGGL(k_dec_2bit, dim3(grid_for(tb.total)), dim3(256), 0, st, c, blob,
+                           reinterpret_cast<const TwoBit*>(blob + tb.items), pre(tb), tb.n);
+    auto scatter = [&](const List& l) {
+        if (l.n)
+            hipLaunchKernelGGL(k_dec_scatter, dim3(grid_for(l.total)), dim3(256), 0, st, c, blob, s32,
+                               reinterpret_cast<const Scatter*>(blob + l.items), pre(l), l.n);
+    };
+    scatter(s1);
+    hipLaunchKernelGGL(k_dec_copy3, dim3(grid_for(n)), dim3(256), 0, st, c, n);
+    if (up.n)
+        hipLaunchKernelGGL(k_dec_unpack, dim3(grid_for(up.total)), dim3(256), 0, st, blob, s32, s64,
+                           reinterpret_cast<const Unpack*>(blob + up.items), pre(up), up.n);
+    scatter(s2);
+    scatter(s3);
+    if (ex.n) {
+        const Expand* items = reinterpret_cast<const Expand*>(blob + ex.items);
+        hipLaunchKernelGGL(k_dec_starts, dim3(ex.n), dim3(1024), 0, st, s32, items);
+        hipLaunchKernelGGL(k_dec_expand, dim3(grid_for(ex.total)), dim3(256), 0, st, c, s32, s64, items, pre(ex), ex.n);
+    }
+    // rows: lengths, block offsets, text
+    const DecWin* wins = reinterpret_cast<const DecWin*>(blob + wins_at);
+    hipLaunchKernelGGL(k_dec_rowlen, dim3((uint32_t)nblk), dim3(256), 0, st, c, blob, wins, (uint32_t)b.wins.size(), n,
                        rowlen, bsum);
     launch_scan_blocks(st, bsum, (uint32_t)nblk, tot);
     uint64_t bytes = 0;
     DECCHK(hipMemcpyAsync(&bytes, tot, 8, hipMemcpyDeviceToHost, st));
     DECCHK(hipStreamSynchronize(st));
-    char* text;
-    DECCHK(m.alloc(&text, bytes));
-    hipLaunchKernelGGL(k_dec_format, dim3((uint32_t)nblk), dim3(256), 0, st, c, blob, d_w, (uint32_t)b.wins.size(), n,
-                       rowlen, bsum, text);
+    if (d.text.n < bytes) DECCHK(d.text.alloc(bytes));
+    hipLaunchKernelGGL(k_dec_format, dim3((uint32_t)nblk), dim3(256), 0, st, c, blob, wins, (uint32_t)b.wins.size(), n,
+                       rowlen, bsum, d.text.p);
     DECCHK(hipGetLastError());
-    std::unique_ptr<char[]> host(new char[bytes ? bytes : 1]);
-    DECCHK(hipMemcpyAsync(host.get(), text, bytes, hipMemcpyDeviceToHost, st));
-    DECCHK(hipStreamSynchronize(st));
-    if (bytes && std::fwrite(host.get(), 1, bytes, fo) != bytes) return fail(GSNP_E_IO, "cannot write " + out);
+    int device = 0;
+    DECCHK(hipGetDevice(&device));
+    d.drain = std::async([&d, device, bytes, &fo, out] { return write_text(d, device, bytes, fo, out); });
     return GSNP_OK;
 }
 
@@ -629,16 +720,11 @@ int decompress_device(const std::string& prefix, const std::string& out)
     std::string err;
     int rc = rd.open(prefix, err);
     if (rc) return fail(rc == 1 ? GSNP_E_IO : GSNP_E_FORMAT, err);
-    FILE* fo = std::fopen(out.c_str(), "w");
-    if (!fo) return fail(GSNP_E_IO, "cannot create " + out);
-    hipStream_t st = nullptr;
-    hipError_t e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
-    if (e != hipSuccess) {
-        std::fclose(fo);
-        return fail(GSNP_E_DEVICE, std::string("hipStreamCreate: ") + hipGetErrorString(e));
-    }
+    OutFile fo(out);
     Batch b;
     RawChunk c;
+    Decoder d;  // goes first: nothing is in flight then
+    DECCHK(d.init());
     bool got = true;
     rc = GSNP_OK;
     while (!rc) {
@@ -649,14 +735,15 @@ int decompress_device(const std::string& prefix, const std::string& out)
         }
         if (got) b.add(c);
         if (!got || b.wins.size() >= 16 || b.sites >= (4u << 20)) {
-            rc = decode_batch(st, b, fo, out);
+            rc = decode_batch(d, b, fo, out);
             b = Batch();
         }
         if (!got) break;
     }
-    (void)hipStreamSynchronize(st);
-    (void)hipStreamDestroy(st);
-    if (std::fclose(fo) != 0 && !rc) rc = fail(GSNP_E_IO, "cannot write " + out);
+    const int w = d.finish();
+    if (!fo.ready()) return fail(GSNP_E_IO, "cannot create " + out);
+    if (w) return w;
+    if (!fo.close() && !rc) rc = fail(GSNP_E_IO, "cannot write " + out);
     return rc;
 }
 
