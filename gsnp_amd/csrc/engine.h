@@ -325,7 +325,8 @@ struct Ctx {
     DevBuf<uint32_t> dict_bits, dict_wpre, dict_out;
     DevBuf<uint64_t> dict_bsum;
     ColBufs cols;  // -C column encoder
-    DevBuf<unsigned long long> calib;  // calibration sub-histograms
+    DevBuf<unsigned long long> calib;  // calibration counts
+    DevBuf<uint32_t> calib_part;       // and each workgroup's
 
     int set_matrix(const double* p_matrix);
     void swap_chrom(ChromState& s);
