@@ -191,38 +191,36 @@ __global__ __launch_bounds__(256) void k_col_count(ColIn in, uint32_t* cnt)
     if (t < kNC) cnt[(size_t)blockIdx.x * kNC + t] = wc[0][t] + wc[1][t] + wc[2][t] + wc[3][t];
 }
 
-// per window: exclusive scan of each counter over the window's blocks
+// per window and counter: exclusive scan over the window's blocks (a window's
+// sixteen counters one after the other in one workgroup took 20 us; 4 us)
 __global__ __launch_bounds__(256) void k_col_scan(const uint32_t* cnt, uint32_t n, uint32_t* boff, uint32_t* tot)
 {
     __shared__ uint32_t wsum[4];
-    const uint32_t w = blockIdx.x, t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const uint32_t w = blockIdx.x, c = blockIdx.y, t = threadIdx.x, lane = t & 63, wv = t >> 6;
     const uint32_t C = min(kWin, n - w * kWin);
     const uint32_t nb = (C + kCB - 1) / kCB;
     const size_t b0 = (size_t)w * kWinBlocks;
-    for (int c = 0; c < kNC; c++) {
-        uint32_t v[4], sum = 0;
-        for (int k = 0; k < 4; k++) {
-            const uint32_t b = t * 4 + k;
-            v[k] = b < nb ? cnt[(b0 + b) * kNC + c] : 0u;
-            sum += v[k];
-        }
-        uint32_t incl = sum;
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t y = __shfl_up(incl, off);
-            if ((int)lane >= off) incl += y;
-        }
-        if (lane == 63) wsum[wv] = incl;
-        __syncthreads();
-        uint32_t run = incl - sum;
-        for (uint32_t k = 0; k < wv; k++) run += wsum[k];
-        for (int k = 0; k < 4; k++) {
-            const uint32_t b = t * 4 + k;
-            if (b < nb) boff[(b0 + b) * kNC + c] = run;
-            run += v[k];
-        }
-        if (t == 255) tot[(size_t)w * kNC + c] = run;
-        __syncthreads();
+    uint32_t v[4], sum = 0;
+    for (int k = 0; k < 4; k++) {
+        const uint32_t b = t * 4 + k;
+        v[k] = b < nb ? cnt[(b0 + b) * kNC + c] : 0u;
+        sum += v[k];
     }
+    uint32_t incl = sum;
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t y = __shfl_up(incl, off);
+        if ((int)lane >= off) incl += y;
+    }
+    if (lane == 63) wsum[wv] = incl;
+    __syncthreads();
+    uint32_t run = incl - sum;
+    for (uint32_t k = 0; k < wv; k++) run += wsum[k];
+    for (int k = 0; k < 4; k++) {
+        const uint32_t b = t * 4 + k;
+        if (b < nb) boff[(b0 + b) * kNC + c] = run;
+        run += v[k];
+    }
+    if (t == 255) tot[(size_t)w * kNC + c] = run;
 }
 
 struct EmitOut {
@@ -1318,14 +1316,22 @@ __global__ __launch_bounds__(256) void k_col_sizes(WriteArgs a, uint32_t nwin)
     }
 }
 
-constexpr uint32_t kWriteParts = 16;  // blocks per chunk
+constexpr uint32_t kWriteGroups = 8;  // a chunk's pieces are dealt to eight groups of blocks
+constexpr uint32_t kWriteSlices = 8;  // blocks of a group, each copying its slice of a piece
+constexpr uint32_t kWriteParts = kWriteGroups * kWriteSlices;
 
-// Block `part` of the chunk's kWriteParts blocks copies its slice of every
-// piece (slices start on 4-byte boundaries); part 0 also writes the headers.
+typedef uint32_t Bytes16 __attribute__((ext_vector_type(4), aligned(1)));
+
+// Block `part` of the chunk's blocks copies its slice of its group's pieces,
+// sixteen bytes a thread at any alignment; part 0 also writes the headers.
+// Bound by the chain of a block's pieces: each waits for its loads.  (With all
+// of the up to 24 pieces in every block, byte by byte where a piece is
+// misaligned, a contig of two windows took 28 us; now 10.)
 struct CopySink {
     uint8_t* dst;
     uint32_t part;
     uint64_t* stage;  // LDS, 8 values
+    uint32_t piece = 0;
     __device__ void vals(const uint64_t* v, int count, uint64_t nbytes)
     {
         if (part == 0) {
@@ -1339,16 +1345,16 @@ struct CopySink {
     }
     __device__ void bytes(const void* p, uint64_t nbytes)
     {
-        const uint8_t* src = static_cast<const uint8_t*>(p);
-        const uint64_t lo = (nbytes * part / kWriteParts) & ~3ull;
-        const uint64_t hi = part + 1 == kWriteParts ? nbytes : (nbytes * (part + 1) / kWriteParts) & ~3ull;
-        if (((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 3) == 0) {
-            const uint64_t q0 = lo / 4, q1 = hi / 4;
+        const uint32_t slice = part / kWriteGroups;
+        if (piece++ % kWriteGroups == part % kWriteGroups) {
+            const uint8_t* src = static_cast<const uint8_t*>(p);
+            const uint64_t lo = (nbytes * slice / kWriteSlices) & ~15ull;
+            const uint64_t hi = slice + 1 == kWriteSlices ? nbytes : (nbytes * (slice + 1) / kWriteSlices) & ~15ull;
+            const uint64_t q0 = lo / 16, q1 = hi / 16;
+#pragma unroll 4
             for (uint64_t q = q0 + threadIdx.x; q < q1; q += blockDim.x)
-                reinterpret_cast<uint32_t*>(dst)[q] = reinterpret_cast<const uint32_t*>(src)[q];
-            for (uint64_t b = q1 * 4 + threadIdx.x; b < hi; b += blockDim.x) dst[b] = src[b];
-        } else {
-            for (uint64_t b = lo + threadIdx.x; b < hi; b += blockDim.x) dst[b] = src[b];
+                *reinterpret_cast<Bytes16*>(dst + 16 * q) = *reinterpret_cast<const Bytes16*>(src + 16 * q);
+            for (uint64_t b = q1 * 16 + threadIdx.x; b < hi; b += blockDim.x) dst[b] = src[b];
         }
         dst += nbytes;
     }
@@ -1471,7 +1477,7 @@ int encode_columns(Ctx& c, uint32_t offset, uint32_t ws_abs, uint32_t n, const C
         in.n = ns;
         c.timer.begin(kStColumns, st);
         hipLaunchKernelGGL(k_col_count, dim3(nblk), dim3(kCB), 0, st, in, b.cnt.p);
-        hipLaunchKernelGGL(k_col_scan, dim3(nwin), dim3(256), 0, st, b.cnt.p, ns, b.boff.p, b.tot.p);
+        hipLaunchKernelGGL(k_col_scan, dim3(nwin, kNC), dim3(256), 0, st, b.cnt.p, ns, b.boff.p, b.tot.p);
         EmitOut eo;
         eo.id4 = b.id4.p, eo.id6 = b.id6.p, eo.idn = b.idn.p, eo.nidx = b.nidx.p;
         eo.x12i = b.x12i.p, eo.x12v = b.x12v.p, eo.x13i = b.x13i.p, eo.x13v = b.x13v.p;
