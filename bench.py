@@ -8,8 +8,8 @@ hits per read, 2% uncovered blocks -- generated in memory by gsnp_amd's seeded
 generator and calibrated on the device.  Every contig's reads stay resident in
 HBM.
 
-A step is one calling pass over every contig: site matrix -> depth classes ->
-fused sort + FP64 likelihood + posterior -> .cns rows formatted on the device
+A step is one calling pass over every contig: depth classes of 64-site tiles ->
+reads to calls (sort, FP64 likelihood, posterior) -> .cns rows formatted on the device
 and copied to pinned host memory, each span's copy running beside the next
 span's kernels.  The timed region starts with the reads in HBM and ends with
 every row in host memory.  Beside it, in the same run: the per-window (plain)
@@ -45,7 +45,7 @@ WORKLOADS = {
     4: "2 Mb reference, 30x 100 bp reads, miscalibrated qualities (delta 3 above q30, cycle offset to 2)",
     5: "248 Mb reference, 30x 150 bp pairs (insert 400+-40), cycle-decaying qualities, rank-sum test",
 }
-TRAFFIC_PROFILE = {3: ROOT / "profiles" / "fused_stage_c3_hbm_traffic.md"}
+TRAFFIC_PROFILE = {3: ROOT / "profiles" / "tiles_c3_hbm_traffic.md"}
 
 
 def host_share() -> int:
@@ -279,7 +279,7 @@ def main() -> int:
                  "batched_over_plain": round(p_secs / secs, 3)}
         print(f"[bench] plain: {p_secs * 1e3:.1f} ms/pass", file=sys.stderr, flush=True)
 
-    # per-stage HIP-event times (eager launches, rows left in HBM)
+    # per-stage HIP-event times (rows left in HBM)
     stage_ms, launches = {}, {}
     if not args.no_stages:
         job.profile(enable=True)
@@ -288,24 +288,24 @@ def main() -> int:
         prof = job.profile(enable=False)
         stage_ms = {k: v[0] / args.steps for k, v in prof.items() if v[1]}
         launches = {k: v[1] / args.steps for k, v in prof.items() if v[1]}
-    # roofline of the dominant stage: the fused sort + likelihood + posterior
-    # (4 B per record read once, 64 B of per-site counters and reference in,
-    # 16 B of calls out: 4n + 80 per site)
-    fused_bytes = 4 * recs + 80 * sites
+    # roofline of the dominant stage: the reads-to-calls launches (a byte per
+    # read base and 8 B of each read's fields in; per site its reference, 64 B
+    # of counters and 16 B of calls)
+    fused_bytes = reads * (args.read_len + 8) + 80 * sites
     roofline = None
     if stage_ms.get("fused"):
         t_f = stage_ms["fused"] / 1e3
         achieved = fused_bytes / t_f / 1e9
         traffic, src = measured_traffic(args.config, args.scale)
         t_call_gbs = fused_bytes / secs / 1e9
-        roofline = {"bound": "hbm", "kernel": "k_fused<S>: sort + likelihood + posterior, one launch per depth class",
+        roofline = {"bound": "hbm", "kernel": "k_call_tile<D>: reads to calls, one launch per depth class",
                     "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic, "traffic_source": src,
                     "bytes_per_pass": int(fused_bytes), "ms_per_pass": round(t_f * 1e3, 4),
                     "spans_per_pass": launches.get("fused"),
-                    "note": "one k_fused launch per depth class and span; achieved is over their HIP-event time",
+                    "note": "the launches of a span from its reads to its calls; achieved is over their HIP-event time",
                     "t_call": {"achieved": round(t_call_gbs, 2), "frac": round(t_call_gbs / HBM_PEAK_GBS, 4),
-                               "note": "the same 4n + 80 bytes per site over the whole timed pass, rows to host"}}
+                               "note": "the same bytes over the whole timed pass, rows to host"}}
 
     # the window build (reads -> records), as its own figure: 2 B per
     # observed base read (base and quality), 4 B per record written, 12 B of

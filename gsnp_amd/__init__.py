@@ -431,7 +431,7 @@ class Job:
         return {s: (ms[i], cnt[i]) for i, s in enumerate(STAGES)}
 
     def autotune(self, start: int = 0, n_sites: int | None = None, reps: int = 2) -> dict:
-        """Tune the fused launch of the batched form on the selected chromosome
+        """Tune the launches per depth class on the selected chromosome
         (gsnp_autotune); returns the chosen shape."""
         if n_sites is None:
             n_sites = self._length - start

@@ -1,6 +1,6 @@
 // walk.h -- dependency-adjusted quality of the sorted records of one site
-// (kernel/likelihood_kernel.cu:168-256).  Shared by the per-window
-// likelihood kernel and the adjoint's record keys.
+// (kernel/likelihood_kernel.cu:168-256), for the likelihood kernel of a
+// caller's records that are not plain.
 #pragma once
 
 #include <hip/hip_runtime.h>
