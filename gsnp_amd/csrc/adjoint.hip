@@ -375,9 +375,10 @@ __global__ __launch_bounds__(256) void k_adj_site(const double* T, const uint32_
 // per piece of up to 256 records, a block took as long as its longest piece:
 // 0.89 ms over 60 million records, 0.79 in chunks).  Workgroups are dealt to
 // the eight XCDs in turn and start in order, so the list of work gives
-// workgroup 8 j + x the j-th share of the site blocks x, x + 8, ...: a block's weights are gathered by one XCD, out of its
-// L2, while few blocks are in flight (waves that stay for the whole launch drift
-// apart over the blocks, and two in three gathers missed: 0.79 ms; this way 0.56).
+// workgroup 8 j + x the j-th share of the site blocks x, x + 8, ...: a block's
+// weights are gathered by one XCD, out of its L2, while few blocks are in flight
+// (waves that stay for the whole launch drift apart over the blocks, and two in
+// three gathers missed: 0.79 ms; this way 0.56).
 // Chunks of 32 and blocks of 8,192 sites are as fast here, but their pieces
 // cost the next kernel 35 to 75 us more.
 constexpr uint32_t kChunksPerGroup = 48;  // of a workgroup
