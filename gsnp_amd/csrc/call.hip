@@ -838,10 +838,11 @@ __global__ __launch_bounds__(256) void k_span_clear(SpanClear clr)
 }
 
 // first read that starts at or after v: a search among the reads of v's
-// kReadBlock sites
+// kReadBlock sites.  The index is that of the last reads loaded, which a
+// chromosome without reads (n = 0) does not have.
 __device__ uint64_t lower_start(const ReadView& r, int64_t v)
 {
-    if (v <= 0) return 0;
+    if (v <= 0 || r.n == 0) return 0;
     const uint64_t k = (uint64_t)v / kReadBlock;
     uint64_t lo = r.first[k], hi = r.first[k + 1];
     while (lo < hi) {

@@ -188,6 +188,7 @@ RefView Ctx::ref_view() const
 ReadView Ctx::read_view() const
 {
     ReadView v;
+    v.n = n_reads;
     v.pos = rpos.p;
     v.meta = rmeta.p;
     v.first = rfirst.p;

@@ -43,6 +43,7 @@ struct RefView {
 
 constexpr uint32_t kReadBlock = 1024;  // sites per entry of ReadView::first
 struct ReadView {
+    uint64_t n = 0;                   // reads of the chromosome; with none, nothing below is read
     const uint64_t* first = nullptr;  // [len / kReadBlock + 3]: first read at or after each block of sites
     const int32_t* pos = nullptr;
     const uint32_t* meta = nullptr;
