@@ -105,9 +105,9 @@ struct FusedArgs {
     int write_lk = 0;   // also store the ten log-likelihoods of each site
     int posterior = 1;  // call the sites (0: likelihoods only, for the per-window path)
     // caller-owned records (posterior 0): sorted rows written back, and the
-    // sites whose records are not all plain (k_likelihood's sites) listed
+    // list entries of the sites that are scored set to kScored; the others'
+    // records are not all plain (k_likelihood's sites)
     int store = 0;
-    uint32_t *odd_list = nullptr, *odd_count = nullptr;
     // the adjoint's record words, each site's from key_off on (key_block: a power of two)
     uint32_t* key_words = nullptr;
     const uint64_t* key_off = nullptr;

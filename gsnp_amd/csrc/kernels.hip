@@ -492,20 +492,37 @@ __device__ __forceinline__ void regs_merge(uint32_t* v, uint32_t lane)
 }
 
 // ---------------------------------------------------------------------------
-// (c) likelihood of listed sites, one thread per site over its sorted records
-// in memory (kernel/likelihood_kernel.cu:168-256): walk_adjusted gives each
-// record's dependency-adjusted quality in record order and the 10 genotype
+// (c) likelihood of the listed sites that k_fused leaves, one thread per site
+// over its sorted records in memory (kernel/likelihood_kernel.cu:168-256):
+// walk_adjusted gives each record's dependency-adjusted quality in record order and the 10 genotype
 // scores of its row (one 128-byte line of the score table) are added in that
 // order.  It takes the records of a caller that k_fused does not: occurrence
 // bytes other than 1, or bits above the base set.
-__global__ __launch_bounds__(256) void k_likelihood(Tables t, SiteArrays a, const uint32_t* list,
-                                                    const uint32_t* list_count, double* lk, uint32_t* err)
+constexpr uint32_t kScored = ~0u;  // list entry of a site that k_fused has scored
+
+__global__ __launch_bounds__(256) void k_likelihood(Tables t, SiteArrays a, const uint32_t* lists, uint32_t pitch,
+                                                    const uint32_t* counts, double* lk, uint32_t* err)
 {
     __shared__ uint32_t seen_all[256 * 17];
     uint32_t* seen = seen_all + threadIdx.x * 17;
-    const uint32_t count = *list_count;
-    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < count; i += gridDim.x * 256u) {
-        const uint32_t s = list[i];
+    uint32_t before[7] = {0};  // entries of the class lists before each
+#pragma unroll
+    for (int k = 0; k < 6; k++) before[k + 1] = before[k] + counts[k];
+    // a wave's lanes lie evenly over the lists: 64 of the deepest sites together
+    // would be the launch's last waves by far
+    const uint32_t waves = (before[6] + 63u) / 64u;
+    for (uint32_t w = blockIdx.x * 4u + (threadIdx.x >> 6); w < waves; w += gridDim.x * 4u) {
+        const uint32_t i = lane_id() * waves + w;
+        if (i >= before[6]) continue;
+        uint32_t cls = 0, at = i;
+#pragma unroll
+        for (uint32_t k = 1; k < 6; k++)
+            if (i >= before[k]) {
+                cls = k;
+                at = i - before[k];
+            }
+        const uint32_t s = lists[(size_t)cls * pitch + at];
+        if (s == kScored) continue;
         const uint32_t n = (uint32_t)a.nrec[s];
         const uint32_t* row = a.rec + (size_t)s * kSlots;
         double acc[10];
@@ -791,6 +808,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(S <= 128 ? 
         const uint64_t key0 = KEYS && act ? f.key_off[site] : 0ull;
         // (a site that is not called has no words)
         const uint32_t n = !act ? 0u : KEYS ? (uint32_t)(f.key_off[site + 1] - key0) : (uint32_t)f.a.nrec[site];
+        uint32_t odd_passes = 0;  // STORE: bit k, my lane group's site of pass k is not plain
+        bool odd_site = false;    // mine is not
         wave_lds_sync();  // the previous group's rows have been read
         // phase 1: sort, dependency counts, score rows parked in LDS
         if constexpr (S <= 64) {
@@ -830,24 +849,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(S <= 128 ? 
 #pragma unroll
                 for (uint32_t k = 0; k < CH; k += 2) bitonic_all2<2, S>(v[k], v[k + 1], e);  // CH is even
                 if constexpr (STORE) {
-                    uint32_t odd = 0;  // bit k: my record of pass k is not plain
+                    bool plain = false;  // one of the chunk's records is of a plain site
                     const bool all_odd = !f.t.qadj_full;
 #pragma unroll
                     for (uint32_t k = 0; k < CH; k++) {
                         const uint32_t st = (uint32_t)__shfl((int)site, (int)((k0 + k) * P + sub));
-                        if (e < nk[k]) {
-                            f.a.rec[(size_t)st * kSlots + e] = v[k];
-                            odd |= all_odd || odd_record(v[k]) ? 1u << k : 0u;
-                        }
+                        const bool mine = e < nk[k];
+                        if (mine) f.a.rec[(size_t)st * kSlots + e] = v[k];
+                        const bool odd = (__ballot(mine && (all_odd || odd_record(v[k]))) & gmask) != 0;
+                        odd_passes |= odd ? 1u << (k0 + k) : 0u;
+                        plain = plain || (mine && !odd);
                     }
-                    if (__ballot(odd != 0)) {
-#pragma unroll 1
-                        for (uint32_t k = 0; k < CH; k++) {
-                            const uint64_t who = __ballot((odd >> k) & 1u) & gmask;
-                            const uint32_t st = (uint32_t)__shfl((int)site, (int)((k0 + k) * P + sub));
-                            if (who && e == 0) f.odd_list[atomicAdd(f.odd_count, 1u)] = st;
-                        }
-                    }
+                    if (!__ballot(plain)) continue;
                 }
 #pragma unroll
                 for (uint32_t k = 0; k < CH; k++) {
@@ -919,6 +932,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(S <= 128 ? 
                     }
                 }
             }
+            if constexpr (STORE)
+                odd_site = ((uint32_t)__shfl((int)odd_passes, (int)(lane % P * S)) >> (lane / P & 31u)) & 1u;
             // (a table with zeros scores every site of a caller's records in k_likelihood, which sees their own)
             if (qf_min == 0u || (!STORE && qa_min == 0u)) bad |= kErrQadjRange;
         } else {
@@ -955,7 +970,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(S <= 128 ? 
                             odd = odd || !f.t.qadj_full || odd_record(v[gi][r]);
                         }
                     }
-                    if (__ballot(odd) && lane == 0) f.odd_list[atomicAdd(f.odd_count, 1u)] = st;
+                    if (__ballot(odd)) {
+                        odd_site = odd_site || lane == gi;
+                        continue;
+                    }
                 }
                 uint32_t slot[R], beyond = 0;
                 wide_slots<R>(v[gi], below, upto, td, gd, bad, slot);
@@ -979,6 +997,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(S <= 128 ? 
             }
         }
         if constexpr (KEYS) continue;
+        uint32_t n_scored = n;
+        if constexpr (STORE) {
+            // the sites left to k_likelihood keep their entries: a list of their
+            // own, appended to with an atomic a site, took 1.5 ms for 200,000
+            const bool scored = act && !odd_site;
+            if (scored) const_cast<uint32_t*>(list)[g0 + lane] = kScored;
+            if (!__ballot(scored)) continue;
+            n_scored = odd_site ? 0u : n;
+        }
         wave_lds_sync();
         // phase 2: twelve sites at a time, lane (sl, cl) adds genotypes 2cl and
         // 2cl+1 of site r * 12 + sl in record order, eight records in flight; the
@@ -988,7 +1015,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(S <= 128 ? 
 #pragma unroll 1
         for (uint32_t r = 0; r < (G + 11) / 12; r++) {
             const uint32_t gi = r * 12u + sl;
-            const uint32_t ng = (uint32_t)__shfl((int)n, (int)(gi & 63u));
+            const uint32_t ng = (uint32_t)__shfl((int)n_scored, (int)(gi & 63u));
             const bool on = lane < 60u && gi < gcount;
             const uint32_t m = on ? ng : 0u;
             const uint32_t* rw = srt + (on ? gi : 0u) * RS;
@@ -1105,18 +1132,19 @@ void launch_fused(hipStream_t st, const FusedArgs& f, const uint32_t* lists, uin
 
 // The sites go through the same launches as the per-window path's, with the
 // sorted rows written back; those with a record that is not plain are scored
-// again from their sorted rows, one thread each.  200,003 sites of mean depth
+// from their sorted rows, one thread each.  200,003 sites of mean depth
 // 30, 1 % of 200-256 records: 3.4 ms with one thread for every site, whose
-// record walk is serial and whose score rows come 16 bytes a lane; 0.25 ms this way.
+// record walk is serial and whose score rows come 16 bytes a lane; 0.25 ms this
+// way.  200,000 sites of depth 30 whose records occur one to three times are as
+// fast as with sort launches before that thread, 0.44 ms, since a group of such
+// sites is only sorted here; scored here as well, and listed by an atomic each,
+// they took 1.93.
 void launch_sort_likelihood(hipStream_t st, const Tables& t, const SiteArrays& a, uint32_t n_sites, uint32_t* lists,
                             uint32_t pitch, uint32_t* counts, double* lk, uint32_t* err, const FusedTune& tune,
                             const uint32_t* skip)
 {
     if (!n_sites) return;
-    launch_fill_u32(st, counts + 6, 1, 0u);
-    // class 0 holds no list of its own: the odd sites' place
-    const uint32_t mc = tune.min_class ? tune.min_class : 1u;
-    launch_bucket(st, a.nrec, n_sites, lists, pitch, counts, 1, nullptr, (int)mc, skip);
+    launch_bucket(st, a.nrec, n_sites, lists, pitch, counts, 1, nullptr, (int)tune.min_class, skip);
     FusedArgs f;
     f.t = t;
     f.a = a;
@@ -1125,14 +1153,10 @@ void launch_sort_likelihood(hipStream_t st, const Tables& t, const SiteArrays& a
     f.write_lk = 1;
     f.posterior = 0;
     f.store = 1;
-    f.odd_list = lists;
-    f.odd_count = counts + 6;
-    FusedTune shape = tune;
-    shape.min_class = mc;
-    launch_fused(st, f, lists, pitch, counts, n_sites, shape);
+    launch_fused(st, f, lists, pitch, counts, n_sites, tune);
     const uint32_t blocks = (n_sites + 255) / 256;
-    hipLaunchKernelGGL(k_likelihood, dim3(blocks < 1024u ? blocks : 1024u), dim3(256), 0, st, t, a, f.odd_list,
-                       f.odd_count, lk, err);
+    hipLaunchKernelGGL(k_likelihood, dim3(blocks < 1024u ? blocks : 1024u), dim3(256), 0, st, t, a, lists, pitch, counts,
+                       lk, err);
 }
 
 void launch_deep_tiles(hipStream_t st, const FusedArgs& f, const ReadView& r, const uint64_t* range, uint32_t n_built,
