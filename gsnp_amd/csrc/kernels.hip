@@ -992,8 +992,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(S <= 128 ? 
 #pragma unroll
                 for (int r = 0; r < R; r++)  // padding slots: row 0, all +0.0
                     srt[gi * RS + (uint32_t)r * 64u + lane] =
-                        slot[r] != 0xFFFFFFFFu ? score_row(f.t.qadj, slot[r], beyond) : 0u;
-                if constexpr (!STORE) bad |= beyond;
+                        slot[r] != 0xFFFFFFFFu ? score_row(f.t.qadj, slot[r], STORE ? beyond : bad) : 0u;
             }
         }
         if constexpr (KEYS) continue;
