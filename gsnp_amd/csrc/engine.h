@@ -199,6 +199,7 @@ struct ChromState {
     DevBuf<uint64_t> rfirst;  // first read at or after each kReadBlock sites
     DevBuf<uint8_t> rseq;  // kSeqFront bytes, the packed reads, kSeqBack bytes
     std::vector<int32_t> h_rpos;
+    std::vector<int64_t> h_tile_gain;
     std::vector<gsnp_snp> h_snps;
     std::vector<uint8_t> h_snp_ref;
 };
@@ -275,6 +276,7 @@ struct Ctx {
     DevBuf<uint64_t> rfirst;
     DevBuf<uint8_t> rseq;
     std::vector<int32_t> h_rpos;
+    std::vector<int64_t> h_tile_gain;  // what the tiles save over the blocks of kReadBlock sites before each (tile_gain)
     // sites of the current window (or batched span)
     uint32_t ws = 0;
     uint32_t win_cap = 0;
@@ -357,6 +359,7 @@ struct Ctx {
     int span_prepare(uint32_t n);
     void span_enqueue(uint32_t start, uint32_t n);
     void span_enqueue_tiles(uint32_t start, uint32_t n);
+    bool span_takes_tiles(uint32_t start, uint32_t n) const;
     FusedArgs fused_args(uint32_t start);
 };
 

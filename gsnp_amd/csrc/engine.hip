@@ -305,6 +305,7 @@ void Ctx::swap_chrom(ChromState& s)
     rfirst.swap(s.rfirst);
     rseq.swap(s.rseq);
     h_rpos.swap(s.h_rpos);
+    h_tile_gain.swap(s.h_tile_gain);
     h_snps.swap(s.h_snps);
     h_snp_ref.swap(s.h_snp_ref);
     built = false;
@@ -516,6 +517,29 @@ static bool is_acgt(char ch)
     }
 }
 
+// Picoseconds that the tile kernels save against the launches per depth class
+// on a block of sites, from the reads that start in it.  With at most 80 reads
+// over a tile of 64 sites on average, nearly every tile runs with 8 to 12 waves
+// a CU.  Beyond 116 most are of the 128-record class, three waves a CU for its
+// 40 KB of LDS each, whose time goes by the reads of a tile: shorter reads, of
+// which a tile holds more at a given depth, lose sooner.  Beyond a depth of 160
+// or 560 reads a tile both ways call most sites by the 256-record network.
+// 1 Mb of uniform depth in us, tiles and launches per class: 100 bp reads 175
+// and 243 at 8x, 298 and 460 at 30x, 397 and 658 at 45x, 1044 and 1051 at 70x,
+// 1625 and 1392 at 100x, 2791 and 2125 at 130x, 3440 and 3294 at 180x; 36 bp
+// reads 511 and 648 at 40x, 1265 and 744 at 52x; 250 bp reads 1313 and 1440 at
+// 100x, 1869 and 1723 at 120x.  8x with a tenth of it at 130x: 561 and 590, with
+// a fifth: 850 and 822.
+static int64_t tile_gain(uint64_t reads, uint32_t sites, uint32_t read_len)
+{
+    const double depth = (double)reads * read_len / sites, over = (double)reads * (read_len + 63) / sites;
+    const double gain = over <= 80.0                    ? 40.0 + 3.0 * over
+                        : over <= 116.0                 ? 80.0
+                        : depth > 160.0 || over > 560.0 ? 0.0
+                                                        : 523.0 + 6.0 * depth - 8.5 * over;
+    return (int64_t)(gain * sites);
+}
+
 int gsnp_load_reads(gsnp_ctx* c, const gsnp_read_batch* b)
 {
     if (!c || !b) return fail(GSNP_E_ARG, "null argument");
@@ -608,6 +632,12 @@ int gsnp_load_reads(gsnp_ctx* c, const gsnp_read_batch* b)
     for (size_t k = 0; k < nfirst; k++) {
         while (at < b->n && (uint64_t)b->pos[at] < (uint64_t)k * kReadBlock) at++;
         first[k] = at;
+    }
+    c->h_tile_gain.assign(nfirst, 0);
+    for (size_t k = 0; k + 1 < nfirst; k++) {
+        const uint64_t a = (uint64_t)k * kReadBlock;
+        const uint64_t sites = a < chr_len ? std::min<uint64_t>(kReadBlock, chr_len - a) : 0;
+        c->h_tile_gain[k + 1] = c->h_tile_gain[k] + (sites ? tile_gain(first[k + 1] - first[k], (uint32_t)sites, L) : 0);
     }
     HIPCHK(c->rfirst.alloc(nfirst));
     HIPCHK(hipMemcpyAsync(c->rfirst.p, first.data(), 8 * nfirst, hipMemcpyHostToDevice, c->stream));
@@ -934,6 +964,14 @@ int gsnp_format_g(double v, char* out)
 
 namespace gsnp {
 
+// The span's blocks together; one without reads takes the tiles.
+bool Ctx::span_takes_tiles(uint32_t start, uint32_t n) const
+{
+    if (!n_reads || !n) return true;
+    const size_t a = start / kReadBlock, b = ((size_t)start + n + kReadBlock - 1) / kReadBlock;
+    return h_tile_gain[b] > h_tile_gain[a];
+}
+
 // Site matrix of the span [start, start+n) straight from the device read
 // store: every read that covers it, no window batches and no carry, with the
 // q_sum of window-boundary sites before their own reads kept in head_qs.
@@ -956,7 +994,7 @@ int Ctx::span_prepare(uint32_t n)
 // and a span's first call a quarter longer for the capture.
 void Ctx::span_enqueue(uint32_t start, uint32_t n)
 {
-    if (tile_ok) {
+    if (tile_ok && span_takes_tiles(start, n)) {
         span_enqueue_tiles(start, n);
         return;
     }
