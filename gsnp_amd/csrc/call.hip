@@ -43,7 +43,9 @@
 // registers and LDS for that many records: 16, 32, 40, 64, 128.  A third of
 // a 30x genome's tiles lie at 33 to 40, and there 12 waves a CU instead of
 // the 64-record class's 8 took the launches from 6.1 to 5.3 ms.  Tiles beyond
-// 128 records a site or 512 reads go through k_site_build and k_fused<256>.
+// 128 records a site or 256 reads go through k_site_build and k_fused<256>, and
+// spans that lie mostly beyond the 64-record class do not come here at all
+// (tile_gain).
 #include <hip/hip_runtime.h>
 
 #include <utility>
@@ -58,7 +60,11 @@ namespace {
 
 constexpr uint32_t kTile = 64;
 constexpr uint32_t kPriorBytes = 640u;   // ten log10 priors of the eight reference codes
-constexpr uint32_t kMaxTileReads = 512;  // eight chunks of 64
+// Four chunks of 64.  A wave walks its tile's reads one after the other, so a
+// few tiles of many reads outlast everything beside them: 1 Mb of 36 bp reads
+// at 8x, a hundredth of it at 100x (300 reads a tile) took 455 us with them in
+// the 128-record class, 393 beyond it; 16 kb so mixed 321 and 251.
+constexpr uint32_t kMaxTileReads = 256;
 constexpr uint32_t kShallowReads = 128;  // the same for the classes up to 64 records
 // Spans of up to this many tiles use the 64- and 128-record classes only: a
 // tile alone takes 30 to 40 us, so a launch does however few its tiles, and
