@@ -838,7 +838,7 @@ __global__ __launch_bounds__(256) void k_span_clear(SpanClear clr)
 {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i < clr.n_heads) clr.head_qs[i] = make_int4(0, 0, 0, 0);
-    if (i < 8) clr.counts[i * kCountStride] = 0;
+    if (i < 8) clr.counts[i * kCountStride] = clr.counts[i] = 0;
     if (i == 8) *clr.job_count = 0;
     if (i == 9) *clr.fix_count = 0;
 }
@@ -973,11 +973,16 @@ void launch_class(hipStream_t st, const TileArgs& f, const uint32_t* list, const
 
 uint32_t tile_min_class(uint32_t n_tiles) { return n_tiles <= kFewTiles ? 3u : 0u; }
 
-void launch_tile_classes(hipStream_t st, const ReadView& r, uint32_t ws, uint32_t n_tiles, uint64_t* range,
-                         uint32_t* lists, uint32_t pitch, const SpanClear& clr)
+void launch_span_clear(hipStream_t st, const SpanClear& clr)
 {
     const uint32_t n = clr.n_heads < 10u ? 10u : clr.n_heads;
     hipLaunchKernelGGL(k_span_clear, dim3((n + 255) / 256), dim3(256), 0, st, clr);
+}
+
+void launch_tile_classes(hipStream_t st, const ReadView& r, uint32_t ws, uint32_t n_tiles, uint64_t* range,
+                         uint32_t* lists, uint32_t pitch, const SpanClear& clr)
+{
+    launch_span_clear(st, clr);
     if (!n_tiles) return;
     const uint32_t mc = tile_min_class(n_tiles);
     constexpr uint32_t K = 8;

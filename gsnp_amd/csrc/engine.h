@@ -199,6 +199,7 @@ struct ChromState {
     DevBuf<uint64_t> rfirst;  // first read at or after each kReadBlock sites
     DevBuf<uint8_t> rseq;  // kSeqFront bytes, the packed reads, kSeqBack bytes
     std::vector<int32_t> h_rpos;
+    std::vector<uint32_t> h_most;
     std::vector<int64_t> h_tile_gain;
     std::vector<gsnp_snp> h_snps;
     std::vector<uint8_t> h_snp_ref;
@@ -276,6 +277,8 @@ struct Ctx {
     DevBuf<uint64_t> rfirst;
     DevBuf<uint8_t> rseq;
     std::vector<int32_t> h_rpos;
+    // per kReadBlock sites: the most reads over the start of one of the block's; empty where the tiles take shallow spans
+    std::vector<uint32_t> h_most;
     std::vector<int64_t> h_tile_gain;  // what the tiles save over the blocks of kReadBlock sites before each (tile_gain)
     // sites of the current window (or batched span)
     uint32_t ws = 0;
@@ -359,6 +362,8 @@ struct Ctx {
     int span_prepare(uint32_t n);
     void span_enqueue(uint32_t start, uint32_t n);
     void span_enqueue_tiles(uint32_t start, uint32_t n);
+    SpanClear span_clear(uint32_t n);
+    uint32_t span_top_class(uint32_t start, uint32_t n) const;
     bool span_takes_tiles(uint32_t start, uint32_t n) const;
     FusedArgs fused_args(uint32_t start);
 };

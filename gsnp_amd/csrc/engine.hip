@@ -305,6 +305,7 @@ void Ctx::swap_chrom(ChromState& s)
     rfirst.swap(s.rfirst);
     rseq.swap(s.rseq);
     h_rpos.swap(s.h_rpos);
+    h_most.swap(s.h_most);
     h_tile_gain.swap(s.h_tile_gain);
     h_snps.swap(s.h_snps);
     h_snp_ref.swap(s.h_snp_ref);
@@ -632,6 +633,12 @@ int gsnp_load_reads(gsnp_ctx* c, const gsnp_read_batch* b)
     for (size_t k = 0; k < nfirst; k++) {
         while (at < b->n && (uint64_t)b->pos[at] < (uint64_t)k * kReadBlock) at++;
         first[k] = at;
+    }
+    c->h_most.assign(c->tile_ok ? 0 : nfirst, 0);
+    for (uint64_t i = 0, j = 0; i < b->n && !c->tile_ok; i++) {
+        while (b->pos[j] + (int64_t)L <= b->pos[i]) j++;
+        uint32_t& m = c->h_most[(size_t)b->pos[i] / kReadBlock];
+        m = std::max(m, (uint32_t)std::min<uint64_t>(i - j + 1, UINT32_MAX));
     }
     c->h_tile_gain.assign(nfirst, 0);
     for (size_t k = 0; k + 1 < nfirst; k++) {
@@ -987,6 +994,31 @@ int Ctx::span_prepare(uint32_t n)
     return GSNP_OK;
 }
 
+constexpr uint32_t kShortSpan = 131072;
+
+// The deepest depth class that a site of the span can fall into: its reads
+// start in its own block of kReadBlock sites or the one before.
+uint32_t Ctx::span_top_class(uint32_t start, uint32_t n) const
+{
+    if (!n_reads || !n) return 0;
+    if (h_most.empty()) return 5;
+    const size_t a = start / kReadBlock, b = ((size_t)start + n - 1) / kReadBlock;
+    uint32_t m = 0;
+    for (size_t k = a ? a - 1 : 0; k <= b; k++) m = std::max(m, h_most[k]);
+    return m <= 8 ? 0u : m <= 16 ? 1u : m <= 32 ? 2u : m <= 64 ? 3u : m <= 128 ? 4u : 5u;
+}
+
+SpanClear Ctx::span_clear(uint32_t n)
+{
+    SpanClear clr;
+    clr.head_qs = head_qs.p;
+    clr.n_heads = n / GSNP_WIN + 2;
+    clr.counts = counts.p;
+    clr.job_count = job_count.p;
+    clr.fix_count = fix_count.p;
+    return clr;
+}
+
 // The device work of one batched span, up to the rank-sum jobs: site matrix,
 // depth classes, fused sort + likelihood + posterior, rank-sum.  Launches
 // only (no copies, no host waits), each queued as it is: replayed as captured
@@ -998,19 +1030,26 @@ void Ctx::span_enqueue(uint32_t start, uint32_t n)
         span_enqueue_tiles(start, n);
         return;
     }
-    launch_fill_u32(stream, head_qs.p, (uint32_t)(4 * (n / GSNP_WIN + 2)), 0u);
+    launch_span_clear(stream, span_clear(n));
     timer.begin(kStSiteBuild, stream);
     launch_site_build(stream, read_view(), 0, n_reads, start, n + 1, INT64_MIN, (int64_t)start + n, 0, site_view(0),
                       head_qs.p, ranges.p);
     timer.end(kStSiteBuild, stream);
-    launch_fill_u32(stream, job_count.p, 1, 0u);
-    launch_fill_u32(stream, fix_count.p, 1, 0u);
     SiteArrays a = site_view(0);
+    FusedTune shape = tune;
+    // No launch for a class that no site can reach, and on short spans none for
+    // 16 records beside the 32-record one: their launches, not their work, are
+    // the time.  100 kb with the adjusted qualities of -g 0.95, us: 73 instead
+    // of 100 at 3x, 98 instead of 121 at 15x, 123 instead of 162 at 30x (as one
+    // captured graph, with launches for every class: 89, 119 and 157).
+    shape.max_class = span_top_class(start, n);
+    if (n <= kShortSpan && shape.max_class > 2 && shape.min_class < 2) shape.min_class = 2;
     timer.begin(kStBucket, stream);
-    launch_bucket(stream, a.nrec, n, lists.p, win_cap, counts.p, 1, stat.p, (int)tune.min_class);
+    launch_bucket(stream, a.nrec, n, lists.p, win_cap, counts.p, 1, stat.p, (int)shape.min_class,
+                  nullptr, false);
     timer.end(kStBucket, stream);
     timer.begin(kStFused, stream);
-    launch_fused(stream, fused_args(start), lists.p, win_cap, counts.p, n, tune);
+    launch_fused(stream, fused_args(start), lists.p, win_cap, counts.p, n, shape);
     timer.end(kStFused, stream);
     if (p.rank_sum_mode) {
         Results res = result_view(0);
@@ -1025,14 +1064,8 @@ void Ctx::span_enqueue(uint32_t start, uint32_t n)
 void Ctx::span_enqueue_tiles(uint32_t start, uint32_t n)
 {
     const uint32_t n_tiles = (n + 1 + 63) / 64;  // one more site is built: the last one's next
-    SpanClear clr;
-    clr.head_qs = head_qs.p;
-    clr.n_heads = n / GSNP_WIN + 2;
-    clr.counts = counts.p;
-    clr.job_count = job_count.p;
-    clr.fix_count = fix_count.p;
     timer.begin(kStBucket, stream);
-    launch_tile_classes(stream, read_view(), start, n_tiles, ranges.p, lists.p, n_tiles, clr);
+    launch_tile_classes(stream, read_view(), start, n_tiles, ranges.p, lists.p, n_tiles, span_clear(n));
     timer.end(kStBucket, stream);
     TileArgs f;
     f.t = tables();

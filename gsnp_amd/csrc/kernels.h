@@ -122,6 +122,7 @@ struct FusedArgs {
 // block for that class and the wide ones, eight for the 32 and 64 classes.
 struct FusedTune {
     uint32_t min_class = 1;
+    uint32_t max_class = 5;  // no site is deeper
     uint32_t wpb[6] = {0, 4, 8, 8, 4, 4};
     uint32_t max_blocks[6] = {8192, 8192, 8192, 8192, 8192, 8192};
 };
@@ -151,13 +152,15 @@ struct TileArgs {
     unsigned long long* n_records = nullptr;
     int write_lk = 0;
 };
-// what the first launch of a span clears: window heads, class counters (8, kCountStride words apart), job counters
+// what the first launch of a span clears: window heads, class counters (the tiles' 8, kCountStride words apart, and the
+// sites' in the first words), job counters
 struct SpanClear {
     int4* head_qs = nullptr;
     uint32_t n_heads = 0;
     uint32_t* counts = nullptr;
     uint32_t *job_count = nullptr, *fix_count = nullptr;
 };
+void launch_span_clear(hipStream_t s, const SpanClear& clr);
 // reads, class and class list (lists[class * pitch]) of each tile of 64 sites
 void launch_tile_classes(hipStream_t s, const ReadView& r, uint32_t ws, uint32_t n_tiles, uint64_t* range,
                          uint32_t* lists, uint32_t pitch, const SpanClear& clr);
@@ -183,7 +186,7 @@ void launch_site_build(hipStream_t s, const ReadView& r, uint64_t r0, uint64_t r
                        uint64_t* range);
 void launch_bucket(hipStream_t s, const int32_t* nrec, uint32_t n_sites, uint32_t* lists, uint32_t list_pitch,
                    uint32_t* counts, int all, unsigned long long* n_records, int min_class = 0,
-                   const uint32_t* skip = nullptr);
+                   const uint32_t* skip = nullptr, bool clear = true);
 // sort and likelihood of caller-owned records (rows of 256): counts (8 words)
 // and lists are working memory; nothing happens when *skip (may be null) is set
 void launch_sort_likelihood(hipStream_t s, const Tables& t, const SiteArrays& a, uint32_t n_sites, uint32_t* lists,

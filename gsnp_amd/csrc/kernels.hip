@@ -359,9 +359,9 @@ __global__ __launch_bounds__(256) void k_bucket(const int32_t* nrec, uint32_t n_
 }
 
 void launch_bucket(hipStream_t st, const int32_t* nrec, uint32_t n_sites, uint32_t* lists, uint32_t pitch,
-                   uint32_t* counts, int all, unsigned long long* n_records, int min_class, const uint32_t* skip)
+                   uint32_t* counts, int all, unsigned long long* n_records, int min_class, const uint32_t* skip, bool clear)
 {
-    launch_fill_u32(st, counts, 6, 0u);
+    if (clear) launch_fill_u32(st, counts, 6, 0u);
     const uint32_t blocks = (n_sites + 256 * kBucketPer - 1) / (256 * kBucketPer);
     if (blocks)
         hipLaunchKernelGGL(k_bucket, dim3(blocks), dim3(256), 0, st, nrec, n_sites, lists, pitch, counts, all,
@@ -1125,7 +1125,7 @@ void launch_fused(hipStream_t st, const FusedArgs& f, const uint32_t* lists, uin
 {
     if (!max_sites) return;
     // deepest classes first: their groups are the longest
-    for (int cls = 5; cls >= (int)tune.min_class; cls--)
+    for (int cls = (int)(tune.max_class > tune.min_class ? tune.max_class : tune.min_class); cls >= (int)tune.min_class; cls--)
         launch_fused_one(st, f, lists, pitch, counts, max_sites, (uint32_t)cls, tune.wpb[cls], tune.max_blocks[cls]);
 }
 
