@@ -43,9 +43,9 @@
 // registers and LDS for that many records: 16, 32, 40, 64, 128.  A third of
 // a 30x genome's tiles lie at 33 to 40, and there 12 waves a CU instead of
 // the 64-record class's 8 took the launches from 6.1 to 5.3 ms.  Tiles beyond
-// 128 records a site or 256 reads go through k_site_build and k_fused<256>, and
-// spans that lie mostly beyond the 64-record class do not come here at all
-// (tile_gain).
+// 128 records a site, 512 reads or max_unique go through k_site_build and
+// k_fused<256>, and spans that lie mostly beyond the 64-record class do not
+// come here at all (tile_gain).
 #include <hip/hip_runtime.h>
 
 #include <utility>
@@ -60,12 +60,21 @@ namespace {
 
 constexpr uint32_t kTile = 64;
 constexpr uint32_t kPriorBytes = 640u;   // ten log10 priors of the eight reference codes
-// Four chunks of 64.  A wave walks its tile's reads one after the other, so a
-// few tiles of many reads outlast everything beside them: 1 Mb of 36 bp reads
-// at 8x, a hundredth of it at 100x (300 reads a tile) took 455 us with them in
-// the 128-record class, 393 beyond it; 16 kb so mixed 321 and 251.
-constexpr uint32_t kMaxTileReads = 256;
+constexpr uint32_t kMaxTileReads = 512;  // eight chunks of 64
 constexpr uint32_t kShallowReads = 128;  // the same for the classes up to 64 records
+// Unique-hit reads a tile may have: of more, most share their anchor with
+// another one, and a wave settles such reads one after the other, so that a few
+// tiles of short reads outlast everything beside them.  A strand has pitch + 63
+// anchors.  16 kb of 36 bp reads at 8x, a thirtieth of it at 100x: 321 us
+// without this limit, 222 with it; 1 Mb with a hundredth so deep 455 and 372.
+// With it at 205 for 100 bp reads, 24 contigs of 0.12 to 2.4 Mb with piles of
+// repeats took 10.6 ms, 10.4 with it at 239 or none; at 150 for 36 bp reads the
+// mixtures above took 5 % more than at 128.
+__device__ __forceinline__ uint32_t max_unique(uint32_t pitch)
+{
+    const uint32_t m = pitch * 7u / 4u + 64u;
+    return m > kShallowReads ? m : kShallowReads;
+}
 // Spans of up to this many tiles use the 64- and 128-record classes only: a
 // tile alone takes 30 to 40 us, so a launch does however few its tiles, and
 // five classes in a row leave most of the device idle.  24 contigs of 0.12 to
@@ -917,6 +926,11 @@ __global__ __launch_bounds__(512) void k_tile_class(ReadView r, uint32_t ws, uin
             const uint32_t most = wave_max((uint32_t)wave_prefix(hist[w][lane]));
             c = most <= 16 ? 0u : most <= 32 ? 1u : most <= 40 ? 2u : most <= 64 ? 3u : most <= 128 ? 4u : kDeepClass;
             if (e - b > kShallowReads && c < 4u) c = 4u;
+            if (e - b > max_unique(r.pitch)) {
+                int mine = rm_hit(meta[k]) == 1 ? 1 : 0;
+                for (uint64_t i = b + 64u + lane; i < e; i += 64) mine += rm_hit(r.meta[i]) == 1 ? 1 : 0;
+                if (lane_of((uint32_t)wave_prefix(mine), 63) > max_unique(r.pitch)) c = kDeepClass;
+            }
             if (c < min_class) c = min_class;
         }
         cls = lane == k ? c : cls;

@@ -522,7 +522,7 @@ static bool is_acgt(char ch)
 // on a block of sites, from the reads that start in it.  With at most 80 reads
 // over a tile of 64 sites on average, nearly every tile runs with 8 to 12 waves
 // a CU.  Beyond 116 most are of the 128-record class, three waves a CU for its
-// 36 KB of LDS each, whose time goes by the reads of a tile: shorter reads, of
+// 40 KB of LDS each, whose time goes by the reads of a tile: shorter reads, of
 // which a tile holds more at a given depth, lose sooner.  Beyond a depth of 160
 // or 560 reads a tile both ways call most sites by the 256-record network.
 // 1 Mb of uniform depth in us, tiles and launches per class: 100 bp reads 175
