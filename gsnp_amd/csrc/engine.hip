@@ -882,6 +882,7 @@ int gsnp_autotune(gsnp_ctx* c, uint32_t start, uint32_t n, int reps, uint32_t* c
     HIPCHK(hipGetLastError());
     rc = c->check_err();
     if (rc) return rc;
+    best_tune.deep_blocks = best_tune.max_blocks[5];
     c->tune = best_tune;
     if (config) {
         config[0] = best_tune.min_class;
@@ -1099,7 +1100,7 @@ void Ctx::span_enqueue_tiles(uint32_t start, uint32_t n)
     if (fork) (void)hipStreamWaitEvent(stream, ev_join, 0);
     launch_deep_tiles(stream, fused_args(start), read_view(), ranges.p, n + 1, n, head_qs.p,
                       lists.p + (size_t)kTileClasses * n_tiles, counts.p + kTileClasses * kCountStride, lists.p + 5 * (size_t)win_cap,
-                      counts.p + (kTileClasses + 1) * kCountStride, n_tiles, stat.p);
+                      counts.p + (kTileClasses + 1) * kCountStride, n_tiles, stat.p, tune);
     timer.end(kStFused, stream);
     if (p.rank_sum_mode) {
         Results res = result_view(0);

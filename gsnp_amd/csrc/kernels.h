@@ -125,6 +125,7 @@ struct FusedTune {
     uint32_t max_class = 5;  // no site is deeper
     uint32_t wpb[6] = {0, 4, 8, 8, 4, 4};
     uint32_t max_blocks[6] = {8192, 8192, 8192, 8192, 8192, 8192};
+    uint32_t deep_blocks = 1024;  // the same for a span's tiles beyond the tile classes: mostly none, so a small grid
 };
 
 // Counters that many blocks add to lie this many words apart.
@@ -173,7 +174,7 @@ void launch_call_tiles(hipStream_t s, const TileArgs& f, const uint32_t* lists, 
 // sorted and called by the 256-record network
 void launch_deep_tiles(hipStream_t s, const FusedArgs& f, const ReadView& r, const uint64_t* range, uint32_t n_built,
                        uint32_t n_sites, int4* head_qs, const uint32_t* tiles, const uint32_t* n_deep, uint32_t* sites,
-                       uint32_t* site_count, uint32_t n_tiles, unsigned long long* n_records);
+                       uint32_t* site_count, uint32_t n_tiles, unsigned long long* n_records, const FusedTune& tune);
 
 // score rows [base][adjusted quality < 64][cycle] from the table by quality, cycle, base
 void launch_tile_scores(hipStream_t s, const double* score, double* tscore, uint32_t cycles);

@@ -1160,14 +1160,14 @@ void launch_sort_likelihood(hipStream_t st, const Tables& t, const SiteArrays& a
 
 void launch_deep_tiles(hipStream_t st, const FusedArgs& f, const ReadView& r, const uint64_t* range, uint32_t n_built,
                        uint32_t n_sites, int4* head_qs, const uint32_t* tiles, const uint32_t* n_deep, uint32_t* sites,
-                       uint32_t* site_count, uint32_t n_tiles, unsigned long long* n_records)
+                       uint32_t* site_count, uint32_t n_tiles, unsigned long long* n_records, const FusedTune& tune)
 {
     if (!n_tiles) return;
     // few tiles are this deep, so the grids stay small and loop
     const uint32_t blocks = n_tiles < 2048u ? n_tiles : 2048u;
     hipLaunchKernelGGL(k_site_build_list, dim3(blocks), dim3(kBuildSites), 0, st, r, range, f.ws, n_built, n_sites, f.a,
                        head_qs, tiles, n_deep, sites, site_count, n_records);
-    launch_fused_class<256>(st, f, sites, site_count, n_sites, 0, 1024u);
+    launch_fused_class<256>(st, f, sites, site_count, n_sites, tune.wpb[5], tune.deep_blocks);
 }
 
 // ---------------------------------------------------------------------------

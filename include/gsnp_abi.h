@@ -187,8 +187,8 @@ int gsnp_window_recycle(gsnp_ctx* ctx);
 int gsnp_batched_call(gsnp_ctx* ctx, uint32_t start, uint32_t n_sites, int emit_text, uint64_t* nbytes);
 
 /* Autotuner of the launches per depth class (the per-window path; in the
- * batched form the deepest sites and adjusted-quality tables too large for its
- * tiles): builds the span's site matrix, then times the fused launch of every
+ * batched form spans of deep reads, the deepest sites of the others, and every
+ * span where the adjusted-quality table is too large for the tiles): builds the span's site matrix, then times the fused launch of every
  * depth class on it for each smallest network width (8, 16, 32: the lowest
  * bucket edge), waves per block (1, 2, 4, 8) and grid cap (512..8192 blocks),
  * and keeps the fastest shape in the context for later calls.  reps timings per candidate, best kept.

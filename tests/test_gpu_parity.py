@@ -79,16 +79,19 @@ def _rows_by_contig(ref: bytes) -> dict:
     return {k: b"".join(v) for k, v in rows.items()}
 
 
-@pytest.mark.parametrize("name", ["c2w3", "stress"])
-def test_tuned_batched_matches_oracle(datasets, name):
+@pytest.mark.parametrize("name,flags", [("c2w3", {}), ("stress", {}), ("c2w3", {"global_dependency": 0.95}),
+                                        ("stress", {"global_dependency": 0.95})])
+def test_tuned_batched_matches_oracle(datasets, tmp_path, name, flags):
     """The launch shape the autotuner keeps (smallest network width, so small
     sites may run on the 32-lane network, waves per block, grid caps) gives the
-    oracle's text: one batched call per contig after tuning."""
+    oracle's text: one batched call per contig and a per-window pass after
+    tuning.  The batched call uses the shape where the adjusted-quality table
+    is too large for the tiles (0.95); with the default table its deepest sites do."""
     import gsnp_amd
 
     ds = datasets(name)
-    parts = _rows_by_contig(ds.oracle_text().read_bytes())
-    job = gsnp_amd.Job(ds.fasta, ds.soap, dbsnp=ds.dbsnp, **ds.flags)
+    parts = _rows_by_contig(ds.oracle_text(**flags).read_bytes())
+    job = gsnp_amd.Job(ds.fasta, ds.soap, dbsnp=ds.dbsnp, **dict(ds.flags, **flags))
     try:
         job.select(0)
         print(f"[parity] {name} tuned {job.autotune(reps=1)}", flush=True)
@@ -99,15 +102,17 @@ def test_tuned_batched_matches_oracle(datasets, name):
             job.call(batched=64)
             out = _job_text(job)
             assert out == want, f"contig {i}: {len(out)} vs {len(want)} bytes"
+        job.write(tmp_path / "windows.cns", batched=0)
+        assert filecmp.cmp(tmp_path / "windows.cns", ds.oracle_text(**flags), shallow=False)
     finally:
         job.close()
 
 
 @pytest.mark.parametrize("name,tune", [("c2w3", False), ("stress", True)])
 def test_batched_replays_match_oracle(datasets, name, tune):
-    """The batched span runs as a captured graph from its second call on; every
-    replay, with eager per-window passes between them (and, with tune, after
-    the autotuner has changed the launch shape), gives the oracle's text."""
+    """A batched call repeated four times, with per-window passes on the same
+    context and buffers between them (and, with tune, after the autotuner has
+    changed the launch shape), gives the oracle's text every time."""
     import gsnp_amd
 
     ds = datasets(name)
@@ -125,8 +130,8 @@ def test_batched_replays_match_oracle(datasets, name, tune):
             for rep in range(4):
                 job.call(batched=64)
                 out = _job_text(job)
-                assert out == want, f"contig {i} replay {rep}: {len(out)} vs {len(want)} bytes"
-                job.call(batched=0)  # eager per-window pass between replays
+                assert out == want, f"contig {i} call {rep}: {len(out)} vs {len(want)} bytes"
+                job.call(batched=0)  # a per-window pass between the calls
     finally:
         job.close()
 
