@@ -327,8 +327,8 @@ __global__ __launch_bounds__(64 * NW) void k_call_tile(TileArgs f, const uint32_
     const uint32_t qwords = f.qtab_bytes / 4u;  // whole 16-byte units
     double* lprior = reinterpret_cast<double*>(lds);
     uint8_t* qtab = lds + kPriorBytes;
-    __shared__ uint32_t block_sum[2];  // records of the block's sites, waves done
-    if (threadIdx.x < 2) block_sum[threadIdx.x] = 0;
+    __shared__ uint32_t block_sum;  // records of the block's sites
+    if (threadIdx.x == 0) block_sum = 0;
     for (uint32_t i = threadIdx.x; i < 80u; i += 64u * NW) lprior[i] = f.t.lprior[i];
     for (uint32_t i = threadIdx.x; i < qwords; i += 64u * NW)
         reinterpret_cast<uint32_t*>(qtab)[i] = reinterpret_cast<const uint32_t*>(f.qtab)[i];
@@ -836,10 +836,9 @@ __global__ __launch_bounds__(64 * NW) void k_call_tile(TileArgs f, const uint32_
     }
     for (int off = 32; off > 0; off >>= 1) records += (uint32_t)__shfl_xor((int)records, off);
     // one global add per block: adds to one address take turns
-    if (lane == 0) {
-        atomicAdd(&block_sum[0], (uint32_t)records);
-        if (atomicAdd(&block_sum[1], 1u) == (uint32_t)NW - 1u) atomicAdd(f.n_records, (unsigned long long)block_sum[0]);
-    }
+    if (lane == 0) atomicAdd(&block_sum, records);
+    __syncthreads();  // every wave of a block with work comes here
+    if (threadIdx.x == 0) atomicAdd(f.n_records, (unsigned long long)block_sum);
 }
 
 // What a span's first launch clears.
