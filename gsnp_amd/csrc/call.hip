@@ -314,6 +314,9 @@ __device__ __forceinline__ uint32_t shape_field(uint32_t w)
     return (w >> 31) ? st9 + ((shape_len(w) - 1u) << 9) + 257u : 0u - st9;
 }
 
+// waves of a block per class: one block takes a CU's LDS (two of 16 records)
+constexpr int kWaves16 = 8, kWaves32 = 12, kWaves40 = 12, kWaves64 = 8, kWaves128 = 3;
+
 template <int D, int NW>
 __global__ __launch_bounds__(64 * NW) void k_call_tile(TileArgs f, const uint32_t* list, const uint32_t* count_ptr)
 {
@@ -966,23 +969,35 @@ __global__ __launch_bounds__(256) void k_tile_scores(const double* score, double
     tscore[i] = score[(size_t)((qa << 10) | (cyc << 2) | o) * kScoreRowStride + k];
 }
 
+// more than 64 KB of dynamic LDS, on the current device
+template <int D, int NW>
+hipError_t allow_class()
+{
+    constexpr uint32_t most = kPriorBytes + kTileQtabMax + NW * wave_lds<D>();
+    static_assert(most <= 163840u, "a CU's LDS");
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(&k_call_tile<D, NW>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)most);
+}
+
 template <int D, int NW>
 void launch_class(hipStream_t st, const TileArgs& f, const uint32_t* list, const uint32_t* count, uint32_t n_tiles,
                   uint32_t per_cu)
 {
     const uint32_t bytes = kPriorBytes + f.qtab_bytes + NW * wave_lds<D>();
-    static_assert(kPriorBytes + kTileQtabMax + NW * wave_lds<D>() <= 163840u, "a CU's LDS");
-    // above 64 KB of dynamic LDS; once per kernel and process is enough, and it is no stream operation
-    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_call_tile<D, NW>),
-                                                          hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                          (int)(kPriorBytes + kTileQtabMax + NW * wave_lds<D>()));
-    (void)allowed;
     uint32_t blocks = (n_tiles + NW - 1) / NW;
     if (blocks > 256u * per_cu) blocks = 256u * per_cu;
     hipLaunchKernelGGL((k_call_tile<D, NW>), dim3(blocks), dim3(64 * NW), bytes, st, f, list, count);
 }
 
 }  // namespace
+
+hipError_t allow_tile_lds()
+{
+    for (hipError_t (*allow)() : {allow_class<64, kWaves64>, allow_class<40, kWaves40>, allow_class<32, kWaves32>,
+                                  allow_class<16, kWaves16>, allow_class<128, kWaves128>})
+        if (const hipError_t e = allow()) return e;
+    return hipSuccess;
+}
 
 uint32_t tile_min_class(uint32_t n_tiles) { return n_tiles <= kFewTiles ? 3u : 0u; }
 
@@ -1015,17 +1030,17 @@ void launch_call_tiles(hipStream_t st, const TileArgs& f, const uint32_t* lists,
 {
     if (!n_tiles) return;
     const uint32_t C = kCountStride;
-    launch_class<64, 8>(st, f, lists + 3 * (size_t)pitch, counts + 3 * C, n_tiles, 1);
+    launch_class<64, kWaves64>(st, f, lists + 3 * (size_t)pitch, counts + 3 * C, n_tiles, 1);
     if (tile_min_class(n_tiles)) return;
-    launch_class<40, 12>(st, f, lists + 2 * (size_t)pitch, counts + 2 * C, n_tiles, 1);
-    launch_class<32, 12>(st, f, lists + 1 * (size_t)pitch, counts + 1 * C, n_tiles, 1);
-    launch_class<16, 8>(st, f, lists + 0 * (size_t)pitch, counts + 0 * C, n_tiles, 2);
+    launch_class<40, kWaves40>(st, f, lists + 2 * (size_t)pitch, counts + 2 * C, n_tiles, 1);
+    launch_class<32, kWaves32>(st, f, lists + 1 * (size_t)pitch, counts + 1 * C, n_tiles, 1);
+    launch_class<16, kWaves16>(st, f, lists + 0 * (size_t)pitch, counts + 0 * C, n_tiles, 2);
 }
 
 void launch_call_deepest(hipStream_t st, const TileArgs& f, const uint32_t* lists, uint32_t pitch,
                          const uint32_t* counts, uint32_t n_tiles)
 {
-    if (n_tiles) launch_class<128, 3>(st, f, lists + 4 * (size_t)pitch, counts + 4 * kCountStride, n_tiles, 1);
+    if (n_tiles) launch_class<128, kWaves128>(st, f, lists + 4 * (size_t)pitch, counts + 4 * kCountStride, n_tiles, 1);
 }
 
 }  // namespace gsnp

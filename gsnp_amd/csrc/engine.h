@@ -360,8 +360,8 @@ struct Ctx {
                     char* out = nullptr);
     int span_build(uint32_t start, uint32_t n);
     int span_prepare(uint32_t n);
-    void span_enqueue(uint32_t start, uint32_t n);
-    void span_enqueue_tiles(uint32_t start, uint32_t n);
+    int span_enqueue(uint32_t start, uint32_t n);
+    int span_enqueue_tiles(uint32_t start, uint32_t n);
     SpanClear span_clear(uint32_t n);
     uint32_t span_top_class(uint32_t start, uint32_t n) const;
     bool span_takes_tiles(uint32_t start, uint32_t n) const;

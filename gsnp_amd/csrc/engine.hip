@@ -363,6 +363,7 @@ int create_ctx(const gsnp_params* p, const double* p_matrix, gsnp_ctx** out)
     c->h_prank = rank_table();
     const std::vector<uint8_t> tq = tile_qadj(qt);
     c->tile_ok = !tq.empty() && tq.size() <= kTileQtabMax;
+    if (c->tile_ok) HIPCHK(allow_tile_lds());
     c->qtab_bytes = c->tile_ok ? (uint32_t)tq.size() : 0u;
     HIPCHK(c->qtab.alloc(tq.size()));
     if (c->tile_ok) HIPCHK(hipMemcpyAsync(c->qtab.p, tq.data(), tq.size(), hipMemcpyHostToDevice, c->stream));
@@ -809,8 +810,8 @@ int gsnp_batched_call(gsnp_ctx* c, uint32_t start, uint32_t n, int emit_text, ui
     if (start % GSNP_WIN) return fail(GSNP_E_ARG, "span must start on a window boundary");
     int rc = c->span_prepare(n);
     if (rc) return rc;
-    c->span_enqueue(start, n);
-    HIPCHK(hipGetLastError());
+    rc = c->span_enqueue(start, n);
+    if (rc) return rc;
     if (c->p.rank_sum_mode) {
         c->fix_offset = 0;
         rc = c->host_fixups();
@@ -1025,12 +1026,9 @@ SpanClear Ctx::span_clear(uint32_t n)
 // only (no copies, no host waits), each queued as it is: replayed as captured
 // graphs the same launches took 7 % longer on 100 kb and 5 % on 24 contigs,
 // and a span's first call a quarter longer for the capture.
-void Ctx::span_enqueue(uint32_t start, uint32_t n)
+int Ctx::span_enqueue(uint32_t start, uint32_t n)
 {
-    if (tile_ok && span_takes_tiles(start, n)) {
-        span_enqueue_tiles(start, n);
-        return;
-    }
+    if (tile_ok && span_takes_tiles(start, n)) return span_enqueue_tiles(start, n);
     launch_span_clear(stream, span_clear(n));
     timer.begin(kStSiteBuild, stream);
     launch_site_build(stream, read_view(), 0, n_reads, start, n + 1, INT64_MIN, (int64_t)start + n, 0, site_view(0),
@@ -1058,11 +1056,13 @@ void Ctx::span_enqueue(uint32_t start, uint32_t n)
         launch_rank(stream, tables(), a, jobs.p, job_count.p, n, res, fixes.p, fix_count.p, stat.p + 1);
         timer.end(kStRank, stream);
     }
+    HIPCHK(hipGetLastError());
+    return GSNP_OK;
 }
 
 // The same through the tile kernels (call.hip): classes of the span's tiles,
 // reads to calls per class, then the few tiles deeper than those classes.
-void Ctx::span_enqueue_tiles(uint32_t start, uint32_t n)
+int Ctx::span_enqueue_tiles(uint32_t start, uint32_t n)
 {
     const uint32_t n_tiles = (n + 1 + 63) / 64;  // one more site is built: the last one's next
     timer.begin(kStBucket, stream);
@@ -1091,13 +1091,17 @@ void Ctx::span_enqueue_tiles(uint32_t start, uint32_t n)
     // few as well (a fork and join costs about as much as their launch)
     const bool fork = n_tiles > 2048;
     if (fork) {
-        (void)hipEventRecord(ev_fork, stream);
-        (void)hipStreamWaitEvent(side, ev_fork, 0);
+        HIPCHK(hipEventRecord(ev_fork, stream));
+        HIPCHK(hipStreamWaitEvent(side, ev_fork, 0));
     }
     launch_call_deepest(fork ? side : stream, f, lists.p, n_tiles, counts.p, n_tiles);
-    if (fork) (void)hipEventRecord(ev_join, side);
+    hipError_t joined = fork ? hipEventRecord(ev_join, side) : hipSuccess;
     launch_call_tiles(stream, f, lists.p, n_tiles, counts.p, n_tiles);
-    if (fork) (void)hipStreamWaitEvent(stream, ev_join, 0);
+    if (fork && joined == hipSuccess) joined = hipStreamWaitEvent(stream, ev_join, 0);
+    if (joined != hipSuccess) {  // what follows on the stream may not start before the side stream is done
+        (void)hipStreamSynchronize(side);
+        return fail(GSNP_E_DEVICE, std::string("join of the deepest tiles: ") + hipGetErrorString(joined));
+    }
     launch_deep_tiles(stream, fused_args(start), read_view(), ranges.p, n + 1, n, head_qs.p,
                       lists.p + (size_t)kTileClasses * n_tiles, counts.p + kTileClasses * kCountStride, lists.p + 5 * (size_t)win_cap,
                       counts.p + (kTileClasses + 1) * kCountStride, n_tiles, stat.p, tune);
@@ -1108,6 +1112,8 @@ void Ctx::span_enqueue_tiles(uint32_t start, uint32_t n)
         launch_rank(stream, tables(), site_view(0), jobs.p, job_count.p, n, res, fixes.p, fix_count.p, stat.p + 1);
         timer.end(kStRank, stream);
     }
+    HIPCHK(hipGetLastError());
+    return GSNP_OK;
 }
 
 int Ctx::span_build(uint32_t start, uint32_t n)

@@ -162,6 +162,7 @@ struct SpanClear {
     uint32_t *job_count = nullptr, *fix_count = nullptr;
 };
 void launch_span_clear(hipStream_t s, const SpanClear& clr);
+hipError_t allow_tile_lds();  // once for each device, before the first launch there
 // reads, class and class list (lists[class * pitch]) of each tile of 64 sites
 void launch_tile_classes(hipStream_t s, const ReadView& r, uint32_t ws, uint32_t n_tiles, uint64_t* range,
                          uint32_t* lists, uint32_t pitch, const SpanClear& clr);
