@@ -559,11 +559,13 @@ static int scan_counts(Ctx& c, const uint32_t* in, uint32_t n, uint64_t* out)
     return GSNP_OK;
 }
 
-// a workspace of at least n elements; kept between spans
+// a workspace of at least n elements, kept between spans; one that a much longer
+// span left behind is given back
 template <class T>
 static hipError_t room(DevBuf<T>& b, size_t n)
 {
-    return b.n < n || !b.p ? b.alloc(n) : hipSuccess;
+    constexpr size_t kept = (size_t(4) << 20) / sizeof(T);  // 4 MB stay whatever the span
+    return b.p && b.n >= n && (b.n <= kept || b.n / 4 <= n) ? hipSuccess : b.alloc(n);
 }
 
 }  // namespace gsnp

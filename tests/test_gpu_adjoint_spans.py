@@ -103,3 +103,39 @@ def test_span_edges_match_autograd(spans, start, size):
     assert abs(float(log_het.grad) - dh) <= 1e-9 * abs(dh) + 1e-13
     again = adj.eval(p0, lh)
     assert np.array_equal(again[1].view(np.uint64), grad.view(np.uint64))
+
+
+def test_a_long_span_s_memory_is_given_back(built):
+    """A span a thousandth as long as the one before it: most of the device memory that the longer one took is free
+    again, and the gradient is that of the short span in a context of its own."""
+    import gsnp_amd
+    from gsnp_amd.adjoint import Adjoint
+
+    hip, free, total = ctypes.CDLL("libamdhip64.so.7"), ctypes.c_size_t(), ctypes.c_size_t()
+
+    def free_bytes():
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    pm = np.full(256 * 256 * 16, 0.02)
+    pm.reshape(256, 256, 4, 4)[:, :, range(4), range(4)] = 0.94
+    job = gsnp_amd.Job(synth=(4, 5, 0.25))  # 500 kb
+    try:
+        job.select(0)
+        job.call(batched=32, emit_text=0)  # the sites' rows, which both share
+        before = free_bytes()
+        Adjoint(job)
+        long = free_bytes()
+        got = Adjoint(job, start=3000, n_sites=500).eval(pm, math.log(1e-3))
+        short = free_bytes()
+    finally:
+        job.close()
+    taken = before - long
+    print(f"[adjoint] long span {taken >> 20} MiB, given back {(short - long) >> 20} MiB", flush=True)
+    assert taken > 200 << 20 and short - long > taken // 2
+    job = gsnp_amd.Job(synth=(4, 5, 0.25))
+    try:
+        ref = Adjoint(job, start=3000, n_sites=500).eval(pm, math.log(1e-3))
+    finally:
+        job.close()
+    assert got[0] == ref[0] and got[2] == ref[2] and np.array_equal(got[1], ref[1])
