@@ -704,6 +704,8 @@ extern "C" int gsnp_adjoint_prepare(gsnp_ctx* c, uint32_t start, uint32_t n)
     launch_fill_u32(st, c->adj_grad.p, 2u * 64u * 256u * 16u, 0u);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(st));
+    c->adj_snps = c->h_snps;
+    c->adj_snp_ref = c->h_snp_ref;
     c->adj_start = start;
     c->adj_n = n;
     c->adj_nrec = nr;
@@ -716,7 +718,9 @@ extern "C" int gsnp_adjoint_prepare(gsnp_ctx* c, uint32_t start, uint32_t n)
 
 // Prior rows (log10) at het rate exp(log_het): the 8 reference-code rows
 // (cpp/prior.cc:3-43), then one row per known SNP (cpp/prior.cc:45-97); and
-// per row the genotypes whose prior carries one factor of het.
+// per row the genotypes whose prior carries one factor of het.  The rows of a
+// prepared span are those of the chromosome it was prepared on.
+static const std::vector<gsnp_snp>& adjoint_snps(const Ctx& c) { return c.adj_n ? c.adj_snps : c.h_snps; }
 static void adjoint_priors(const Ctx& c, double log_het, std::vector<double>& lp, std::vector<uint32_t>& mask)
 {
     gsnp_params pp = c.p;
@@ -729,12 +733,14 @@ static void adjoint_priors(const Ctx& c, double log_het, std::vector<double>& lp
     for (int g = 0; g < 10; g++)
         if ((kGenoCodes[g] >> 2) != (kGenoCodes[g] & 3)) het_bits |= 1u << g;
     mask.assign(8, het_bits);
-    const size_t nsnp = c.h_snps.size();
+    const std::vector<gsnp_snp>& snps = adjoint_snps(c);
+    const std::vector<uint8_t>& snp_ref = c.adj_n ? c.adj_snp_ref : c.h_snp_ref;
+    const size_t nsnp = snps.size();
     lp.resize((8 + nsnp) * 10);
     mask.resize(8 + nsnp);
     for (size_t i = 0; i < nsnp; i++) {
-        const gsnp_snp& sn = c.h_snps[i];
-        snp_log_prior(pp, prior.data(), c.h_snp_ref[i], sn, &lp[(8 + i) * 10]);
+        const gsnp_snp& sn = snps[i];
+        snp_log_prior(pp, prior.data(), snp_ref[i], sn, &lp[(8 + i) * 10]);
         uint32_t m = 0;
         for (int g = 0; g < 10; g++) {
             const int a1 = kGenoCodes[g] >> 2, a2 = kGenoCodes[g] & 3;
@@ -798,7 +804,7 @@ extern "C" int gsnp_adjoint_info(gsnp_ctx* c, uint32_t* n_sites, uint64_t* n_rec
     if (!c) return fail(GSNP_E_ARG, "null context");
     if (n_sites) *n_sites = c->adj_n;
     if (n_records) *n_records = c->adj_nrec;
-    if (n_prior_rows) *n_prior_rows = 8 + (uint32_t)c->h_snps.size();
+    if (n_prior_rows) *n_prior_rows = 8 + (uint32_t)adjoint_snps(*c).size();
     return GSNP_OK;
 }
 

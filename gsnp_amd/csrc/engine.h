@@ -320,6 +320,8 @@ struct Ctx {
     // key within each block of sites, the reduction pieces and the keys in use
     uint32_t adj_start = 0, adj_n = 0, adj_npieces = 0, adj_nblk = 0, adj_nuk = 0, adj_groups = 0;
     uint64_t adj_nrec = 0;
+    std::vector<gsnp_snp> adj_snps;  // known SNPs of the span's chromosome, which the prior rows count through
+    std::vector<uint8_t> adj_snp_ref;
     DevBuf<uint32_t> adj_cnt, adj_prow, adj_word, adj_sword, adj_tmp, adj_hist, adj_hbase, adj_cbase, adj_cpiece, adj_mask;
     DevBuf<uint32_t> adj_pstart, adj_pblock, adj_kpiece, adj_used, adj_ukey;
     DevBuf<uint64_t> adj_off, adj_start_of, adj_pidx, adj_uidx, adj_hoff, adj_bsum;

@@ -139,3 +139,50 @@ def test_a_long_span_s_memory_is_given_back(built):
     finally:
         job.close()
     assert got[0] == ref[0] and got[2] == ref[2] and np.array_equal(got[1], ref[1])
+
+
+def test_a_prepared_span_outlives_its_chromosome(built):
+    """The context gets a chromosome without known SNPs after a span with some was prepared: the span's evaluation
+    still has its own prior rows."""
+    import gsnp_amd
+
+    lib, check = gsnp_amd.lib(), gsnp_amd.check
+    rng = np.random.default_rng(3)
+    n, k = 3000, 900
+    codes = rng.integers(0, 4, n).astype(np.uint8)
+    at = np.sort(rng.choice(n, k, replace=False)).astype(np.uint32)
+    codes[at] |= 8
+    snps = (gsnp_amd.Snp * k)()
+    for s, f in zip(snps, rng.dirichlet(np.ones(4), k)):
+        s.hapmap, s.validated = 1, 1
+        s.freq[:] = f
+    pos = np.sort(rng.integers(0, n - L - 1, 1200)).astype(np.int32)
+    m = len(pos)
+    arrays = (pos, np.full(m, (L << 16) | 1, np.int32), np.full(m, ord("+"), np.uint8),
+              np.frombuffer(b"ACTG", np.uint8)[codes[pos[:, None] + np.arange(L)] & 3], np.full((m, L), 64 + 30, np.uint8))
+    rb = gsnp_amd.ReadBatch(m, L, *(a.ctypes.data for a in arrays))
+    pm = np.full(256 * 256 * 16, 0.02)
+    pm.reshape(256, 256, 4, 4)[:, :, range(4), range(4)] = 0.94
+    p, ctx = gsnp_amd.params(read_length=L, refine_mode=1), ctypes.c_void_p()
+    check(lib.gsnp_device_init(0))
+    check(lib.gsnp_create(ctypes.byref(p), pm.ctypes.data, ctypes.byref(ctx)))
+    try:
+        def evaluate():
+            ll, dh, g, sites, rows = ctypes.c_double(), ctypes.c_double(), np.zeros(64 * 256 * 16), np.zeros(n), ctypes.c_uint32()
+            check(lib.gsnp_adjoint_eval(ctx, pm.ctypes.data, math.log(1e-3), ctypes.byref(ll), g.ctypes.data,
+                                        ctypes.byref(dh), sites.ctypes.data))
+            check(lib.gsnp_adjoint_info(ctx, None, None, ctypes.byref(rows)))
+            return ll.value, dh.value, g, sites, rows.value
+
+        check(lib.gsnp_set_chromosome(ctx, b"a", codes.ctypes.data, n, at.ctypes.data, ctypes.addressof(snps), k))
+        check(lib.gsnp_load_reads(ctx, ctypes.byref(rb)))
+        check(lib.gsnp_adjoint_prepare(ctx, 0, n))
+        first = evaluate()
+        assert first[4] == 8 + k
+        other = np.zeros(500, np.uint8)
+        check(lib.gsnp_set_chromosome(ctx, b"b", other.ctypes.data, 500, None, None, 0))
+        second = evaluate()
+        assert first[:2] == second[:2] and first[4] == second[4]
+        assert np.array_equal(first[2], second[2]) and np.array_equal(first[3], second[3])
+    finally:
+        lib.gsnp_destroy(ctx)
