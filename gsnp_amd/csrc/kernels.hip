@@ -745,9 +745,6 @@ __host__ __device__ constexpr uint32_t qadj_lds_words(uint32_t td, uint32_t gd)
     return ((64u * td * gd + 15u) / 16u) * 4u;  // whole 16-byte units
 }
 
-// Up to 128 records the kernel is held to 128 VGPRs, four waves per SIMD
-// (the 64-record class would take 148 and three waves; with four, the
-// stage is about 3 % faster); the 256 class keeps its registers.
 // The adjoint's word of a record: its score row (16 bits for an adjusted
 // quality below 64, the gradient table's) and its site within a block of sites.
 __device__ __forceinline__ uint32_t key_word(uint32_t row, uint32_t site, uint32_t block, uint32_t& bad)
@@ -766,6 +763,9 @@ __device__ __forceinline__ bool odd_record(uint32_t w) { return (w & 0xFE0000FFu
 // and the sorted rows, or the adjoint's record words.
 enum FusedMode : int { kFusedCall = 0, kFusedScore, kFusedStore, kFusedKeys };
 
+// Up to 128 records the kernel is held to 128 VGPRs, four waves per SIMD
+// (the 64-record class would take 148 and three waves; with four, the
+// stage is about 3 % faster); the 256 class keeps its registers.
 template <int S, bool QL, int MODE>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(S <= 128 ? 4 : 1, 8))) void k_fused(FusedArgs f, const uint32_t* list, const uint32_t* count_ptr)
 {
