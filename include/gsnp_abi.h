@@ -180,8 +180,9 @@ int gsnp_window_results(gsnp_ctx* ctx, uint32_t call_length, const gsnp_window_o
 int gsnp_window_recycle(gsnp_ctx* ctx);
 
 /* Batched form: call sites [start, start+n_sites) of the chromosome straight
- * from the device read store in one fused launch per depth bucket, without
- * the per-window recycle; emit_text formats the rows.  Same outputs as the
+ * from the device read store, by tiles of 64 sites in one launch per depth
+ * class (spans of deep reads: site matrix, then one sorting launch per depth
+ * class), without the per-window recycle; emit_text formats the rows.  Same outputs as the
  * per-window path (no reference counterpart; it replaces the window loop of
  * Call_win::new_soap2cns, cpp/call_genotype.cc:474-644). */
 int gsnp_batched_call(gsnp_ctx* ctx, uint32_t start, uint32_t n_sites, int emit_text, uint64_t* nbytes);

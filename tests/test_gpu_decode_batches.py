@@ -40,3 +40,26 @@ def test_batches_give_the_same_text(built, tmp_path, contigs, length):
     assert a == (tmp_path / "dev.cns").read_bytes()
     with pytest.raises(gsnp_amd.GsnpError, match="cannot create"):
         gsnp_amd.decompress(tmp_path / "cols", tmp_path / "none" / "dev.cns", device=True)
+
+
+@pytest.mark.parametrize("lengths", [[40] * 16 + [3000], [40] * 16 + [60000] * 3, [30000] * 16 + [40] * 17 + [45000]])
+def test_batches_of_growing_text(built, tmp_path, lengths):
+    """Batches of little text, which is written in one copy, before and after ones that go through the pinned pieces."""
+    import gsnp_amd
+
+    rng = random.Random(len(lengths))
+    ref, lines = [], []
+    for c, n in enumerate(lengths):
+        seq = "".join(rng.choices("ACGT", k=n))
+        ref.append(f">c{c}\n{seq}\n")
+        p = rng.randrange(n - 30)
+        lines.append(f"r\t{seq[p:p + 30]}\t{'^' * 30}\t1\ta\t30\t+\tc{c}\t{p + 1}\t0\n")
+    (tmp_path / "g.fa").write_text("".join(ref))
+    (tmp_path / "d.soap").write_text("".join(lines))
+    job = gsnp_amd.Job(tmp_path / "g.fa", tmp_path / "d.soap", read_length=30)
+    job.write(tmp_path / "cols", compress=True, batched=32)
+    job.close()
+    gsnp_amd.decompress(tmp_path / "cols", tmp_path / "dev.cns", device=True)
+    gsnp_amd.decompress(tmp_path / "cols", tmp_path / "host.cns", device=False)
+    text = (tmp_path / "dev.cns").read_bytes()
+    assert text.count(b"\n") == sum(lengths) and text == (tmp_path / "host.cns").read_bytes()
