@@ -45,7 +45,7 @@
 // the 64-record class's 8 took the launches from 6.1 to 5.3 ms.  Tiles beyond
 // 128 records a site, 512 reads or max_unique go through k_site_build and
 // k_fused<256>, and spans that lie mostly beyond the 64-record class do not
-// come here at all (tile_gain).
+// come here at all (add_tile_gain).
 #include <hip/hip_runtime.h>
 
 #include <utility>
@@ -60,21 +60,6 @@ namespace {
 
 constexpr uint32_t kTile = 64;
 constexpr uint32_t kPriorBytes = 640u;   // ten log10 priors of the eight reference codes
-constexpr uint32_t kMaxTileReads = 512;  // eight chunks of 64
-constexpr uint32_t kShallowReads = 128;  // the same for the classes up to 64 records
-// Unique-hit reads a tile may have: of more, most share their anchor with
-// another one, and a wave settles such reads one after the other, so that a few
-// tiles of short reads outlast everything beside them.  A strand has pitch + 63
-// anchors.  16 kb of 36 bp reads at 8x, a thirtieth of it at 100x: 321 us
-// without this limit, 222 with it; 1 Mb with a hundredth so deep 455 and 372.
-// With it at 205 for 100 bp reads, 24 contigs of 0.12 to 2.4 Mb with piles of
-// repeats took 10.6 ms, 10.4 with it at 239 or none; at 150 for 36 bp reads the
-// mixtures above took 5 % more than at 128.
-__device__ __forceinline__ uint32_t max_unique(uint32_t pitch)
-{
-    const uint32_t m = pitch * 7u / 4u + 64u;
-    return m > kShallowReads ? m : kShallowReads;
-}
 // Spans of up to this many tiles use the 64- and 128-record classes only: a
 // tile alone takes 30 to 40 us, so a launch does however few its tiles, and
 // five classes in a row leave most of the device idle.  24 contigs of 0.12 to

@@ -179,6 +179,12 @@ struct ColBufs {
     }
 };
 
+// What the tile kernels save over some tiles (add_tile_gain), the tiles, and
+// their slowness together, in hundredths.
+struct TileGain {
+    int64_t ns = 0, tiles = 0, slow = 0;
+};
+
 // The device inputs of one chromosome: reference codes, known SNPs and the
 // packed read store.  The context holds the selected chromosome's in its own
 // fields; a job that keeps every chromosome resident parks the others in
@@ -200,7 +206,7 @@ struct ChromState {
     DevBuf<uint8_t> rseq;  // kSeqFront bytes, the packed reads, kSeqBack bytes
     std::vector<int32_t> h_rpos;
     std::vector<uint32_t> h_most;
-    std::vector<int64_t> h_tile_gain;
+    std::vector<TileGain> h_tile_gain;
     std::vector<gsnp_snp> h_snps;
     std::vector<uint8_t> h_snp_ref;
 };
@@ -279,7 +285,7 @@ struct Ctx {
     std::vector<int32_t> h_rpos;
     // per kReadBlock sites: the most reads over the start of one of the block's; empty where the tiles take shallow spans
     std::vector<uint32_t> h_most;
-    std::vector<int64_t> h_tile_gain;  // what the tiles save over the blocks of kReadBlock sites before each (tile_gain)
+    std::vector<TileGain> h_tile_gain;  // before each kReadBlock sites; empty where no span takes the tiles
     // sites of the current window (or batched span)
     uint32_t ws = 0;
     uint32_t win_cap = 0;

@@ -519,27 +519,48 @@ static bool is_acgt(char ch)
     }
 }
 
-// Picoseconds that the tile kernels save against the launches per depth class
-// on a block of sites, from the reads that start in it.  With at most 80 reads
-// over a tile of 64 sites on average, nearly every tile runs with 8 to 12 waves
-// a CU.  Beyond 116 most are of the 128-record class, three waves a CU for its
-// 40 KB of LDS each, whose time goes by the reads of a tile: shorter reads, of
-// which a tile holds more at a given depth, lose sooner.  Beyond a depth of 160
-// or 560 reads a tile both ways call most sites by the 256-record network.
-// 1 Mb of uniform depth in us, tiles and launches per class: 100 bp reads 175
-// and 243 at 8x, 298 and 460 at 30x, 397 and 658 at 45x, 1044 and 1051 at 70x,
-// 1625 and 1392 at 100x, 2791 and 2125 at 130x, 3440 and 3294 at 180x; 36 bp
-// reads 511 and 648 at 40x, 1265 and 744 at 52x; 250 bp reads 1313 and 1440 at
-// 100x, 1869 and 1723 at 120x.  8x with a tenth of it at 130x: 561 and 590, with
-// a fifth: 850 and 822.
-static int64_t tile_gain(uint64_t reads, uint32_t sites, uint32_t read_len)
+// Adds to g what the tile kernels save, in nanoseconds, against the launches per
+// depth class on the tile of sites [p0, p0 + 64), whose reads are [b, e), and how
+// slow the tile is by itself.  Tiles of up to 64 records a site run 8 to
+// 12 waves a CU; the 128-record class three, for its 40 KB of LDS each, and its
+// time goes by the reads of a tile, the more so where most share their start;
+// deeper tiles call all their sites by the 256-record network.  The launches per
+// class go by the depth.  1 Mb of uniform depth in us, tiles and launches per
+// class: 100 bp reads 175 and 243 at 8x, 298 and 460 at 30x, 397 and 658 at 45x,
+// 1044 and 1051 at 70x, 1625 and 1392 at 100x, 2791 and 2125 at 130x, 3440 and
+// 3294 at 180x; 36 bp reads 511 and 648 at 40x, 1250 and 695 at 46x; 250 bp reads
+// 1313 and 1440 at 100x, 1869 and 1723 at 120x.  A locus of 100 bp reads every
+// 500 sites: 298 and 285 with 60 reads on one start, 537 and 420 with 100, 766
+// and 470 with 120 on 20 starts, 1184 and 912 with 250.
+static void add_tile_gain(TileGain& g, int64_t weight, const int32_t* pos, uint64_t b, uint64_t e, int64_t p0, uint32_t L)
 {
-    const double depth = (double)reads * read_len / sites, over = (double)reads * (read_len + 63) / sites;
-    const double gain = over <= 80.0                    ? 40.0 + 3.0 * over
-                        : over <= 116.0                 ? 80.0
-                        : depth > 160.0 || over > 560.0 ? 0.0
-                                                        : 523.0 + 6.0 * depth - 8.5 * over;
-    return (int64_t)(gain * sites);
+    const double over = (double)(e - b);
+    double gain = 0.0027 * over - 0.01;  // a site
+    double slow = 0;
+    if (over > 32.0) {
+        uint64_t same = 0, most = 0, bases = 0;  // reads on the start before theirs; most over a site; their bases in the tile
+        for (uint64_t i = b, j = b; i < e; i++) {
+            const int64_t from = std::max<int64_t>(pos[i], p0), to = std::min<int64_t>((int64_t)pos[i] + L, p0 + 64);
+            bases += (uint64_t)(to - from);
+            same += i > b && pos[i] == pos[i - 1];
+            while ((int64_t)pos[j] + L <= from) j++;
+            most = std::max(most, i - j + 1);
+        }
+        const bool piled = 4 * same > 3 * (e - b);
+        const double depth = (double)bases / 64;
+        const double per_class = 0.0145 * std::min(depth, 100.0) + 0.024 * std::max(depth - 100.0, 0.0);
+        const bool beyond = most > 64 || e - b > kShallowReads;
+        if (beyond) slow = std::min(2.0, std::max(0.0, (over - 90.0) / 50.0));
+        if (most > 128 || e - b > kMaxTileReads || e - b > max_unique(L))
+            gain = per_class - (1.7 + 0.0095 * depth);
+        else if (beyond)
+            gain = per_class - (0.0105 * over - 0.1 + (piled ? 0.4 : 0.0));
+        else if (piled)
+            gain = -0.2;
+    }
+    g.ns += (int64_t)(gain * 64.0 * (double)weight);
+    g.tiles += weight;
+    g.slow += (int64_t)(100.0 * slow) * weight;
 }
 
 int gsnp_load_reads(gsnp_ctx* c, const gsnp_read_batch* b)
@@ -627,25 +648,33 @@ int gsnp_load_reads(gsnp_ctx* c, const gsnp_read_batch* b)
     c->h_rpos.assign(b->pos, b->pos + b->n);
     HIPCHK(c->rpos.alloc(b->n + 1));
     HIPCHK(c->rmeta.alloc(b->n + 1));
-    // first read at or after each block of sites (the tiles' range searches)
+    // first read at or after each block of sites (the tiles' range searches),
+    // and what the tiles save before each: all tiles of a short chromosome, one in
+    // four of a longer one
     const size_t nfirst = (size_t)(chr_len / kReadBlock) + 3;
     std::vector<uint64_t> first(nfirst);
-    uint64_t at = 0;
+    c->h_tile_gain.assign(c->tile_ok ? nfirst : 0, TileGain());
+    uint64_t at = 0, covers = 0;  // first read that starts at or after the tile's end, and that covers the tile or starts behind it
+    TileGain gain;
+    const uint32_t every = chr_len <= GSNP_WIN ? 1 : 4;
     for (size_t k = 0; k < nfirst; k++) {
-        while (at < b->n && (uint64_t)b->pos[at] < (uint64_t)k * kReadBlock) at++;
+        const int64_t p = (int64_t)k * kReadBlock;
+        while (at < b->n && b->pos[at] < p) at++;
         first[k] = at;
+        if (!c->tile_ok) continue;
+        c->h_tile_gain[k] = gain;
+        for (uint32_t t = k % every; t < kReadBlock / 64 && p + 64 * t < (int64_t)chr_len; t += every) {
+            const int64_t p0 = p + 64 * t;
+            while (at < b->n && b->pos[at] < p0 + 64) at++;
+            while (covers < at && (int64_t)b->pos[covers] + L <= p0) covers++;
+            add_tile_gain(gain, every, b->pos, covers, at, p0, L);
+        }
     }
     c->h_most.assign(c->tile_ok ? 0 : nfirst, 0);
     for (uint64_t i = 0, j = 0; i < b->n && !c->tile_ok; i++) {
         while (b->pos[j] + (int64_t)L <= b->pos[i]) j++;
         uint32_t& m = c->h_most[(size_t)b->pos[i] / kReadBlock];
         m = std::max(m, (uint32_t)std::min<uint64_t>(i - j + 1, UINT32_MAX));
-    }
-    c->h_tile_gain.assign(nfirst, 0);
-    for (size_t k = 0; k + 1 < nfirst; k++) {
-        const uint64_t a = (uint64_t)k * kReadBlock;
-        const uint64_t sites = a < chr_len ? std::min<uint64_t>(kReadBlock, chr_len - a) : 0;
-        c->h_tile_gain[k + 1] = c->h_tile_gain[k] + (sites ? tile_gain(first[k + 1] - first[k], (uint32_t)sites, L) : 0);
     }
     HIPCHK(c->rfirst.alloc(nfirst));
     HIPCHK(hipMemcpyAsync(c->rfirst.p, first.data(), 8 * nfirst, hipMemcpyHostToDevice, c->stream));
@@ -973,12 +1002,15 @@ int gsnp_format_g(double v, char* out)
 
 namespace gsnp {
 
-// The span's blocks together; one without reads takes the tiles.
+// What the span's blocks save together, and 45 us more, which the fewer launches
+// of the tiles save whatever the span (100 kb at 8x: 54 us and 110, at 60x 158
+// and 225), less the slow tiles' latency (100 kb at 100x: 384 and 324).
 bool Ctx::span_takes_tiles(uint32_t start, uint32_t n) const
 {
     if (!n_reads || !n) return true;
-    const size_t a = start / kReadBlock, b = ((size_t)start + n + kReadBlock - 1) / kReadBlock;
-    return h_tile_gain[b] > h_tile_gain[a];
+    const TileGain &a = h_tile_gain[start / kReadBlock], &b = h_tile_gain[((size_t)start + n + kReadBlock - 1) / kReadBlock];
+    const double slow = 0.01 * (double)(b.slow - a.slow) / (double)std::max<int64_t>(1, b.tiles - a.tiles);
+    return (double)(b.ns - a.ns) + 45000.0 * (1.0 - 1.4 * slow) > 0;
 }
 
 // Site matrix of the span [start, start+n) straight from the device read

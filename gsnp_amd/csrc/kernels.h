@@ -134,6 +134,21 @@ constexpr uint32_t kCountStride = 64;
 // Arguments of the reads-to-calls launch over tiles of 64 sites (call.hip).
 constexpr uint32_t kTileClasses = 5;         // at most 16, 32, 40, 64, 128 records a site; then the deep tiles
 constexpr uint32_t kTileQtabMax = 17408;     // bytes of the adjusted-quality table that fit beside the waves' LDS
+constexpr uint32_t kMaxTileReads = 512;  // eight chunks of 64
+constexpr uint32_t kShallowReads = 128;  // the same for the classes up to 64 records
+// Unique-hit reads a tile may have: of more, most share their anchor with
+// another one, and a wave settles such reads one after the other, so that a few
+// tiles of short reads outlast everything beside them.  A strand has pitch + 63
+// anchors.  16 kb of 36 bp reads at 8x, a thirtieth of it at 100x: 321 us
+// without this limit, 222 with it; 1 Mb with a hundredth so deep 455 and 372.
+// With it at 205 for 100 bp reads, 24 contigs of 0.12 to 2.4 Mb with piles of
+// repeats took 10.6 ms, 10.4 with it at 239 or none; at 150 for 36 bp reads the
+// mixtures above took 5 % more than at 128.
+__host__ __device__ inline uint32_t max_unique(uint32_t pitch)
+{
+    const uint32_t m = pitch * 7u / 4u + 64u;
+    return m > kShallowReads ? m : kShallowReads;
+}
 struct TileArgs {
     Tables t;
     RefView ref;

@@ -18,11 +18,10 @@ N = 12_000
 @pytest.mark.parametrize("read_len,depth,deep,tiles", [
     (100, 30, None, True), (100, 60, None, True), (100, 110, None, False), (100, 220, None, False),
     (36, 40, None, True), (36, 60, None, False), (36, 100, None, False), (200, 90, None, True), (200, 150, None, False),
-    (100, 20, (130, 1000), True), (100, 20, (130, 6000), False), (100, 3, (700, 300), False), (36, 8, (110, 600), True)])
+    (100, 20, (130, 1000), True), (100, 20, (130, 6000), False), (100, 3, (700, 300), True), (36, 8, (110, 600), True)])
 @pytest.mark.parametrize("rank", [0, 1])
 def test_route_and_text(built, tmp_path, read_len, depth, deep, tiles, rank):
-    """deep: (depth, sites) of a part of the chromosome.  The choice goes by means over blocks of 1,024 sites: 300 sites
-    at 700x are two of the twelve blocks at about 80x and 130x.  600 sites of 36 bp reads at 110x are tiles of some 300
+    """deep: (depth, sites) of a part of the chromosome.  600 sites of 36 bp reads at 110x are tiles of some 300
     unique-hit reads in a span that stays with the tiles."""
     import gsnp_amd
 
