@@ -900,7 +900,9 @@ __global__ __launch_bounds__(512) void k_tile_class(ReadView r, uint32_t ws, uin
             const int64_t p0 = (int64_t)ws + (int64_t)tile * kTile;
             hist[w][lane] = 0;
             wave_lds_sync();
+            int uniq = 0;  // my unique-hit reads
             auto count = [&](int32_t p, uint32_t m) {
+                uniq += rm_hit(m) == 1 ? 1 : 0;
                 const int32_t st = (int32_t)((int64_t)p - p0), en = st + (int32_t)rm_len(m);
                 if (rm_hit(m) == 1 && en > 0) {
                     atomicAdd(&hist[w][st > 0 ? st : 0], 1);
@@ -913,11 +915,7 @@ __global__ __launch_bounds__(512) void k_tile_class(ReadView r, uint32_t ws, uin
             const uint32_t most = wave_max((uint32_t)wave_prefix(hist[w][lane]));
             c = most <= 16 ? 0u : most <= 32 ? 1u : most <= 40 ? 2u : most <= 64 ? 3u : most <= 128 ? 4u : kDeepClass;
             if (e - b > kShallowReads && c < 4u) c = 4u;
-            if (e - b > max_unique(r.pitch)) {
-                int mine = rm_hit(meta[k]) == 1 ? 1 : 0;
-                for (uint64_t i = b + 64u + lane; i < e; i += 64) mine += rm_hit(r.meta[i]) == 1 ? 1 : 0;
-                if (lane_of((uint32_t)wave_prefix(mine), 63) > max_unique(r.pitch)) c = kDeepClass;
-            }
+            if (e - b > max_unique(r.pitch) && lane_of((uint32_t)wave_prefix(uniq), 63) > max_unique(r.pitch)) c = kDeepClass;
             if (c < min_class) c = min_class;
         }
         cls = lane == k ? c : cls;
