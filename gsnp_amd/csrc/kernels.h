@@ -138,17 +138,13 @@ constexpr uint32_t kMaxTileReads = 512;  // eight chunks of 64
 constexpr uint32_t kShallowReads = 128;  // the same for the classes up to 64 records
 // Unique-hit reads a tile may have: of more, most share their anchor with
 // another one, and a wave settles such reads one after the other, so that a few
-// tiles of short reads outlast everything beside them.  A strand has pitch + 63
-// anchors.  16 kb of 36 bp reads at 8x, a thirtieth of it at 100x: 321 us
-// without this limit, 222 with it; 1 Mb with a hundredth so deep 455 and 372.
-// With it at 205 for 100 bp reads, 24 contigs of 0.12 to 2.4 Mb with piles of
-// repeats took 10.6 ms, 10.4 with it at 239 or none; at 150 for 36 bp reads the
-// mixtures above took 5 % more than at 128.
-__host__ __device__ inline uint32_t max_unique(uint32_t pitch)
-{
-    const uint32_t m = pitch * 7u / 4u + 64u;
-    return m > kShallowReads ? m : kShallowReads;
-}
+// tiles of short reads outlast everything beside them.  36 bp reads, us: 16 kb at
+// 8x with a thirtieth of it at 100x 319 without the limit, 262 with it; 1 Mb with
+// a hundredth so deep 457 and 398, as much at 40x throughout 513 and 514 (with the
+// limit at 127 a handful of its tiles went past the class, 581).  100 bp reads: 24
+// contigs of 0.12 to 2.4 Mb with piles of repeats 10.4 ms as without it, 11.2 with a
+// limit of 256 on all of a tile's reads.
+__host__ __device__ inline uint32_t max_unique(uint32_t pitch) { return pitch / 2u + 192u; }
 struct TileArgs {
     Tables t;
     RefView ref;
